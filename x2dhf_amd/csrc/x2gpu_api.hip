@@ -1,5 +1,6 @@
 // Context, memory and grid management of the x2gpu C ABI.
 #include "x2gpu_internal.h"
+#include "x2gpu_chain.h"
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -407,6 +408,8 @@ extern "C" int x2g_grid_create(x2g_ctx *ctx, int nni, int nmu, const double *coe
     alloc((void **)&g->vxisq, nmu * sizeof(double));
     alloc((void **)&g->veta, nni * sizeof(double));
     alloc((void **)&g->vetasq, nni * sizeof(double));
+    const size_t rown = (size_t)8 * (nmu + kRowPadLo + kRowPadHi);
+    for (auto &w : g->rowc) alloc((void **)&w, rown * sizeof(float));
     if (rc) {
         x2g_grid_destroy(g);
         return rc;
@@ -423,6 +426,17 @@ extern "C" int x2g_grid_create(x2g_ctx *ctx, int nni, int nmu, const double *coe
     for (int nu = 0; nu < nni; ++nu) {
         dn[nu] = suppl[2 * n + nu];
         dnf[nu] = (float)dn[nu];
+    }
+    // row weights of the chained sweep: row mu at index mu + kRowPadLo
+    for (int kind = 0; kind < 2; ++kind) {
+        std::vector<float> w(rown, 0.0f);
+        for (int mu = 1; mu <= nmu; ++mu)
+            for (int k = 0; k < 4; ++k) {
+                const float c2 = (float)coef[4 + k], bc = (float)(kind == 0 ? bo : bp)[mu - 1] * (float)coef[k];
+                w[8 * (size_t)(mu + kRowPadLo) + k] = c2 + bc;
+                w[8 * (size_t)(mu + kRowPadLo) + 4 + k] = c2 - bc;
+            }
+        if (!rc) rc = x2g_h2d(ctx, g->rowc[kind], w.data(), rown * sizeof(float));
     }
     if (!rc) rc = x2g_h2d(ctx, g->suppl, suppl, 14 * n * sizeof(double));
     if (!rc) rc = x2g_h2d(ctx, g->bmu_orb, bo.data(), nmu * sizeof(double));
@@ -450,6 +464,8 @@ extern "C" int x2g_grid_destroy(x2g_grid *g)
     void *ptrs[] = {g->suppl, g->bmu_orb, g->bmu_pot, g->dnu, g->bmu_orb_f, g->bmu_pot_f,
                     g->dnu_f, g->vxi, g->vxisq, g->veta, g->vetasq};
     for (void *p : ptrs)
+        if (p) x2g_free(c, p);
+    for (float *p : g->rowc)
         if (p) x2g_free(c, p);
     for (auto &kv : g->levels) {
         if (kv.second.off) x2g_free(c, kv.second.off);

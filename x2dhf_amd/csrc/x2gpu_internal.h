@@ -119,6 +119,9 @@ struct x2g_grid {
     double *bmu_orb = nullptr;     // b(mu) for orbitals  (borb(1,mu))
     double *bmu_pot = nullptr;     // b(mu) for potentials (bpot(1,mu))
     double *dnu = nullptr;         // d(nu)  (d(nu,1))
+    // weights of the rows mu-4..mu-1, mu+1..mu+4 in the sweep's operator,
+    // c2 +- b(mu) c1, in FP32, 8 per row, row mu at mu + kRowPadLo; by bkind
+    float *rowc[2] = {nullptr, nullptr};
     float *bmu_orb_f = nullptr, *bmu_pot_f = nullptr, *dnu_f = nullptr;
     double *vxi = nullptr, *vxisq = nullptr, *veta = nullptr, *vetasq = nullptr;
     size_t n() const { return (size_t)nni * nmu; }

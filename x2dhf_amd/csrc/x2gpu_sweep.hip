@@ -27,6 +27,7 @@
 //    each workgroup walks a balanced list of strips (row segments) across
 //    the batch's problems.
 #include "x2gpu_internal.h"
+#include "x2gpu_chain.h"
 #include <algorithm>
 #include <string>
 #include <atomic>
@@ -1432,6 +1433,7 @@ struct CorrDesc {
     const float *e;     // padded FP32 correction
     int nni, nmu;
     int ps;             // row stride of e
+    int groups, first;  // of a chain's rows (ChainOut), else 0
 };
 
 // u += e over the relaxed points, a row per workgroup at a time (row
@@ -1445,7 +1447,12 @@ __global__ void __launch_bounds__(256) k_correct(const CorrDesc *__restrict__ cd
     const gdptr_w u = gmem_w(d.fun);
     for (int r = blockIdx.x; r < rows; r += gridDim.x) {
         const int ub = (1 + r) * nni + 1, eb = (5 + r) * s1 + 5;
-        for (int c = threadIdx.x; c < w; c += blockDim.x) u[ub + c] += (double)e[eb + c];
+        if (d.groups) {
+            for (int c = threadIdx.x; c < w; c += blockDim.x)
+                u[ub + c] += (double)e[eb - 5 + chain_elem(d.groups, d.first + 1 + c / 5, c % 5)];
+        } else {
+            for (int c = threadIdx.x; c < w; c += blockDim.x) u[ub + c] += (double)e[eb + c];
+        }
     }
 }
 
@@ -1996,7 +2003,7 @@ static void fill_desc(SweepDesc<T> &d, x2g_grid *g, const T *lhs, const T *rhs, 
 template <typename T>
 static int pad_row_stride(int nni, int kind)
 {
-    return kind == 2 ? sweep_row_stride(nni, sweep_vec<T>()) : nni + 8;
+    return kind == 3 ? chain_row(chain_groups(nni)) : kind == 2 ? sweep_row_stride(nni, sweep_vec<T>()) : nni + 8;
 }
 
 // Build the even/odd descriptor lists of a batch; a_bufs/b_bufs are the
@@ -3009,7 +3016,26 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
         if (!ordered(it)) (it.prec ? maxnni32 : maxnni64) = std::max(it.prec ? maxnni32 : maxnni64, g->nni);
     }
     const int kind64 = maxnni64 ? sweep_kind<double>(ctx, maxnni64) : 0;
-    const int kind32 = maxnni32 ? sweep_kind<float>(ctx, maxnni32) : 0;
+    int kind32 = maxnni32 ? sweep_kind<float>(ctx, maxnni32) : 0;
+    // kind 3: the FP32 items, those of a grid and b(mu) together, as chains
+    // where that is faster (and no engine or cut is asked for)
+    std::vector<int> i64, i32, iord;  // item indices by precision; ordered (MC)SOR items
+    std::vector<ChainProblem> chain;
+    ChainCut cut{};
+    if (kind32 == 2 && env_engine() == 0 && env_strip_l() <= 0 && !g_plan_fixed && maxsor2 > 0) {
+        for (int i = 0; i < n; ++i)
+            if (items[i].prec) i32.push_back(i);
+        std::stable_sort(i32.begin(), i32.end(), [&](int x, int y) {
+            const x2g_relax_item &p = items[x], &q = items[y];
+            return p.grid_index != q.grid_index ? p.grid_index < q.grid_index : p.bkind < q.bkind;
+        });
+        for (int i : i32) {
+            const x2g_relax_item &it = items[i];
+            chain.push_back({grids[it.grid_index], it.bkind, it.isym, it.omega, nullptr, nullptr, nullptr, nullptr});
+        }
+        if (chain_pays(ctx, chain, maxsor2, cut)) kind32 = 3;
+        else i32.clear();
+    }
     auto pstride = [&](int i) {
         x2g_grid *g = grids[items[i].grid_index];
         return items[i].prec ? pad_row_stride<float>(g->nni, kind32) : pad_row_stride<double>(g->nni, kind64);
@@ -3024,7 +3050,7 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
         return (size_t)2 * split_size(g->nni, g->nmu) * (items[i].prec ? sizeof(float) : sizeof(double));
     };
     size_t off64 = 0, off32 = 0;
-    std::vector<size_t> o64(n), o32(n);
+    std::vector<size_t> o64(n), o32(n), olr(n);
     for (int i = 0; i < n; ++i) {
         x2g_grid *g = grids[items[i].grid_index];
         o64[i] = off64;
@@ -3033,17 +3059,33 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
             off64 += align256(padbytes(i));
         else if (items[i].prec == 0)
             off64 += 2 * align256(padbytes(i)) + align256(lrbytes(i));
-        else
+        else if (kind32 != 3)
             off32 += 2 * align256(padbytes(i)) +
                      2 * align256(std::max<size_t>(g->n(), split_size(g->nni, g->nmu)) * sizeof(float));
+    }
+    // Chained items: all A areas, all B areas, all pairs (read up to kRowPadLo
+    // rows below an item's own, which are areas of others, and up to as many
+    // above, which are others' or follow the last).
+    size_t chain_area = 0;
+    if (kind32 == 3) {
+        for (int i : i32) {
+            o32[i] = chain_area;
+            chain_area += align256(padbytes(i));
+        }
+        off32 = 2 * chain_area;
+        for (int i : i32) {
+            olr[i] = off32;
+            off32 += align256(lrbytes(i));
+        }
+        off32 += (size_t)2 * kRowPadLo * 10 * chain_groups(maxnni32) * sizeof(float);
     }
     if (off64 && (rc = ws_reserve(ctx, 0, off64))) return rc;
     if (off32 && (rc = ws_reserve(ctx, 3, off32))) return rc;
     char *w64 = (char *)ctx->ws[0].ptr;
     char *w32 = (char *)ctx->ws[3].ptr;
 
-    std::vector<int> i64, i32, iord;  // item indices by precision; ordered (MC)SOR items
-    for (int i = 0; i < n; ++i) (ordered(items[i]) ? iord : items[i].prec ? i32 : i64).push_back(i);
+    for (int i = 0; i < n; ++i)
+        if (!items[i].prec || kind32 != 3) (ordered(items[i]) ? iord : items[i].prec ? i32 : i64).push_back(i);
 
     auto bufA = [&](int i) { return (double *)(w64 + o64[i]); };
     auto bufB = [&](int i) { return (double *)(w64 + o64[i] + align256(padbytes(i))); };
@@ -3052,6 +3094,7 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
     // pairs, which extend over the region of k = 3), 3 res_f
     auto f32p = [&](int i, int k) {
         x2g_grid *g = grids[items[i].grid_index];
+        if (kind32 == 3) return (float *)(w32 + (k <= 1 ? o32[i] + k * chain_area : olr[i]));
         const size_t pp = align256(padbytes(i));
         const size_t nn = align256(std::max<size_t>(g->n(), split_size(g->nni, g->nmu)) * sizeof(float));
         size_t o = o32[i] + (k <= 1 ? k * pp : 2 * pp + (k - 2) * nn);
@@ -3161,6 +3204,7 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
 
     // FP32 items: conversion, residual, sweeps, correction
     SweepPlan<float> p32;
+    ChainPlan c32;
     const SweepDesc<float> *d32e = nullptr, *d32o = nullptr;
     const ResDesc *d_res = nullptr;
     const CorrDesc *d_corr = nullptr;
@@ -3196,17 +3240,19 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
             r.rf[2] = it.rhs_f1_d ? it.rhs_f3_d : nullptr;
             r.bmu = it.bkind == 0 ? g->bmu_orb : g->bmu_pot;
             r.dnu = g->dnu;
-            r.res_f = kind32 == 2 ? f32p(i, 2) : f32p(i, 3);
-            r.res_split = kind32 == 2;  // k_sweep: (omega/lhs, r) pairs, formed here each macro-iteration
+            r.res_f = kind32 >= 2 ? f32p(i, 2) : f32p(i, 3);
+            r.res_split = kind32 >= 2;  // k_sweep: (omega/lhs, r) pairs, formed here each macro-iteration
             r.omega = it.omega;
             r.part = nullptr;
             for (int q = 0; q < 16; ++q) r.c[q] = g->coef[q];
             r.nni = g->nni;
             r.nmu = g->nmu;
             res.push_back(r);
-            corr.push_back({it.fun_d, f32p(i, 0), g->nni, g->nmu, pstride(i)});
+            corr.push_back({it.fun_d, f32p(i, 0), g->nni, g->nmu, pstride(i), 0, 0});
             cvt.push_back({it.lhs_d, f32p(i, 2), (long)g->n()});
-            if (kind32 == 2) {
+            if (kind32 == 3) {
+                // every row a chained sweep reads was written by its call
+            } else if (kind32 == 2) {
                 // the correction starts from zero: the first sweep takes A as
                 // zero without reading it, and k_sweep writes every row of
                 // its destination except the mu <= 1 and mu >= nmu-3 rows,
@@ -3232,18 +3278,34 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
                 base[k].lr = f32p(i32[k], 2);
                 base[k].lr_bytes = (unsigned)lrbytes(i32[k]);
             }
-        SweepKnobs kn32;
-        if ((rc = tuned_knobs<float>(ctx, base, A, B, true, kn32))) return rc;
-        plan_sweeps(ctx, base, A, B, p32, &kn32);
-        // the strip engines ping-pong: an odd sweep count leaves the correction in B
-        if (p32.kind != 0 && (maxsor2 % 2) == 1)
-            for (size_t k = 0; k < i32.size(); ++k) corr[k].e = f32p(i32[k], 1);
-        const bool split32 = p32.kind == 2;
-        if ((rc = stage_plan(ctx, p32, &d32e, &d32o))) return rc;
+        if (kind32 == 3) {
+            for (size_t k = 0; k < i32.size(); ++k) {
+                chain[k].lr = f32p(i32[k], 2);
+                chain[k].A = f32p(i32[k], 0);
+                chain[k].B = f32p(i32[k], 1);
+            }
+            if ((rc = chain_plan(ctx, chain, maxsor2, cut, c32))) return rc;
+            for (size_t k = 0; k < i32.size(); ++k) {
+                const ChainOut &o = c32.out[k];
+                corr[k].e = o.e;
+                corr[k].ps = chain_row(o.groups);
+                corr[k].groups = o.groups;
+                corr[k].first = o.first;
+            }
+        } else {
+            SweepKnobs kn32;
+            if ((rc = tuned_knobs<float>(ctx, base, A, B, true, kn32))) return rc;
+            plan_sweeps(ctx, base, A, B, p32, &kn32);
+            // the strip engines ping-pong: an odd sweep count leaves the correction in B
+            if (p32.kind != 0 && (maxsor2 % 2) == 1)
+                for (size_t k = 0; k < i32.size(); ++k) corr[k].e = f32p(i32[k], 1);
+            if ((rc = stage_plan(ctx, p32, &d32e, &d32o))) return rc;
+        }
+        const bool split32 = kind32 >= 2;
         if ((rc = stage_descs(ctx, res, doff, &d_res))) return rc;
         if ((rc = stage_descs(ctx, corr, doff, &d_corr))) return rc;
         if ((rc = stage_descs(ctx, cvt, doff, &d_cvt))) return rc;
-        if ((rc = stage_descs(ctx, zero, doff, &d_zero))) return rc;
+        if (!zero.empty() && (rc = stage_descs(ctx, zero, doff, &d_zero))) return rc;
         nzero = (int)zero.size();
         for (auto &z : zero) maxzero = std::max(maxzero, z.n);
         for (auto &r : res) res_prod = res_prod || r.rf[0];
@@ -3289,9 +3351,13 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
         if (!i32.empty() && maxsor2 > 0) {
             const int n32 = (int)i32.size();
             if ((rc = launch_residual(ctx, d_res, n32, maxnni, maxnmu, maxn, res_prod))) return rc;
-            X2G_LAUNCH(ctx, k_zero_f32, dim3(std::min(grid_x_for(maxzero, 256), 128), nzero), dim3(256), 0, d_zero);
-            X2G_HIP(hipGetLastError());
-            if ((rc = launch_sweeps<float>(ctx, d32e, d32o, p32, maxsor2, /*a_zero=*/true))) return rc;
+            if (kind32 == 3) {
+                if ((rc = chain_run(ctx, c32))) return rc;
+            } else {
+                X2G_LAUNCH(ctx, k_zero_f32, dim3(std::min(grid_x_for(maxzero, 256), 128), nzero), dim3(256), 0, d_zero);
+                X2G_HIP(hipGetLastError());
+                if ((rc = launch_sweeps<float>(ctx, d32e, d32o, p32, maxsor2, /*a_zero=*/true))) return rc;
+            }
             X2G_LAUNCH(ctx, k_correct, dim3((int)std::min<long>(maxnmu, 1024), n32), dim3(256), 0, d_corr);
             X2G_HIP(hipGetLastError());
             X2G_LAUNCH(ctx, k_boundary_fun, dim3(grid_x_for(2 * maxn / std::max<long>(maxnni, 1) + maxnni, 256), n32),

@@ -45,10 +45,11 @@ struct x2g_ctx {
     hipStream_t stream = nullptr;
     int num_cu = 0;
     size_t max_lds = 0;
-    x2g::Workspace ws[6];          // 0: padded work buffers, 1: reduction partials,
+    x2g::Workspace ws[7];          // 0: padded work buffers, 1: reduction partials,
                                    // 2: launch descriptors, 3: FP32 staging,
                                    // 4: padded buffers of batched quadratures,
-                                   // 5: batched reduction partials
+                                   // 5: batched reduction partials,
+                                   // 6: arrays by level of ordered sweeps
     void *pinned = nullptr;        // pinned host staging for descriptors/results
     size_t pinned_bytes = 0;
     void *pinned_out = nullptr;    // pinned host buffer for gathered results
@@ -80,7 +81,7 @@ struct x2g_ctx {
     struct GraphEntry {
         hipGraphExec_t exec = nullptr;
         void *arena = nullptr;
-        void *ws0 = nullptr, *ws3 = nullptr;  // workspace the graph addresses
+        void *ws0 = nullptr, *ws3 = nullptr, *ws6 = nullptr;  // workspace the graph addresses
         long last_use = 0;
     };
     bool graphs_on = false;

@@ -28,6 +28,7 @@
 //    the batch's problems.
 #include "x2gpu_internal.h"
 #include "x2gpu_chain.h"
+#include "x2gpu_front.h"
 #include <algorithm>
 #include <string>
 #include <atomic>
@@ -1975,6 +1976,8 @@ static int set_lds_attr(x2g_ctx *ctx)
         (const void *)k_sweep<float, 1, 528, 2>,
         (const void *)k_sweep<float, 2, 768, 2>};
     for (const void *k : ks) X2G_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, mx));
+    const int rc = front_lds_attr(ctx);
+    if (rc) return rc;
     done = true;
     return X2G_OK;
 }
@@ -2947,6 +2950,13 @@ extern "C" int x2g_relax_ordered(x2g_grid *g, int isym, int bkind, double *work_
     X2G_CHECK(ordering >= X2G_ORDER_COLWISE && ordering <= X2G_ORDER_MIDDLE2,
               "x2g_relax_ordered: ordering must be one of X2G_ORDER_*");
     if (nsweeps == 0) return X2G_OK;
+    if (levels_pipe() && front_fits(g->ctx, g->nni, g->nmu, method, ordering)) {
+        const std::vector<FrontItem> fv = {{g, work_d, lhs_d, rhs_d, omega, bkind, isym, method, ordering}};
+        if (front_reserve(g->ctx, fv, nsweeps) == X2G_OK) {
+            if ((rc = set_lds_attr(g->ctx))) return rc;
+            return launch_fronts(g->ctx, fv, nsweeps);
+        }
+    }
     const x2g_levels *L;
     if ((rc = grid_levels(g, method, ordering, &L))) return rc;
     std::vector<LevelDesc> v(1);
@@ -3186,17 +3196,33 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
     const PadDesc *d_pout64 = nullptr;
     if (!pout64.empty() && (rc = stage_descs(ctx, pout64, doff, &d_pout64))) return rc;
 
-    // ordered (MC)SOR items: level schedules, putout descriptors
+    // ordered (MC)SOR items: fronts or level schedules, putout descriptors
     std::vector<LevelDesc> lev;
+    std::vector<FrontItem> fronts;
+    auto as_front = [&](int i) {
+        const x2g_grid *g = grids[items[i].grid_index];
+        return levels_pipe() && front_fits(ctx, g->nni, g->nmu, items[i].method, items[i].ordering);
+    };
+    for (int i : iord)
+        if (as_front(i)) {
+            const x2g_relax_item &it = items[i];
+            fronts.push_back({grids[it.grid_index], bufA(i), it.lhs_d, it.rhs_d, it.omega, it.bkind, it.isym,
+                              it.method, it.ordering});
+        }
+    // (level schedules take less memory)
+    if (!fronts.empty() && maxsor2 > 0 && front_reserve(ctx, fronts, maxsor2) != X2G_OK) fronts.clear();
+    const bool fronts_on = !fronts.empty();
     std::vector<PadDesc> pout_ord;
     for (int i : iord) {
         const x2g_relax_item &it = items[i];
         x2g_grid *g = grids[it.grid_index];
-        const x2g_levels *L;
-        if ((rc = grid_levels(g, it.method, it.ordering, &L))) return rc;
-        LevelDesc d{};
-        fill_level_desc(d, g, L, bufA(i), it.lhs_d, it.rhs_d, it.bkind, it.isym, it.omega);
-        lev.push_back(d);
+        if (!(fronts_on && as_front(i))) {
+            const x2g_levels *L;
+            if ((rc = grid_levels(g, it.method, it.ordering, &L))) return rc;
+            LevelDesc d{};
+            fill_level_desc(d, g, L, bufA(i), it.lhs_d, it.rhs_d, it.bkind, it.isym, it.omega);
+            lev.push_back(d);
+        }
         pout_ord.push_back({it.fun_d, bufA(i), nullptr, g->nni, g->nmu, 1, g->nni + 8});
     }
     const PadDesc *d_pout_ord = nullptr;
@@ -3342,6 +3368,7 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
         }
         if (!iord.empty() && maxsor2 > 0) {
             if ((rc = launch_levels(ctx, lev, maxsor2))) return rc;
+            if ((rc = launch_fronts(ctx, fronts, maxsor2))) return rc;
             X2G_LAUNCH(ctx, k_putout, dim3(grid_x_for(maxn, 256), (int)iord.size()), dim3(256), 0,
                                d_pout_ord);
             X2G_HIP(hipGetLastError());
@@ -3398,6 +3425,7 @@ static std::string relax_signature(x2g_ctx *ctx, x2g_grid *const *grids, const x
     put(g_plan_gen.load());
     put(ctx->ws[0].ptr);
     put(ctx->ws[3].ptr);
+    put(ctx->ws[6].ptr);
     for (int i = 0; i < n; ++i) {
         const x2g_relax_item &it = items[i];
         const x2g_grid *g = grids[it.grid_index];
@@ -3486,6 +3514,7 @@ static int relax_capture(x2g_ctx *ctx, const std::string &key, x2g_grid *const *
         g.arena = arena;
         g.ws0 = ctx->ws[0].ptr;
         g.ws3 = ctx->ws[3].ptr;
+        g.ws6 = ctx->ws[6].ptr;
         ++ctx->graph_captures;
         *out = &g;
         return X2G_OK;

@@ -170,6 +170,49 @@ __device__ __forceinline__ gdptr gmem(const double *p) { return (gdptr)p; }
 __device__ __forceinline__ gdptr_w gmem_w(double *p) { return (gdptr_w)p; }
 __device__ __forceinline__ gfptr gmem(const float *p) { return (gfptr)p; }
 
+// The arithmetic of a col-wise MCSOR sweep, its roundings spelled out: the
+// kernels that share it give the same result bit for bit, whichever of them a
+// batch's sizes choose.
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// Weight of a row mu -+ k: c2 +- b(mu) c1.
+template <typename T>
+__device__ __forceinline__ T mcsor_row_weight(T b, T c1, T c2)
+{
+#pragma clang fp contract(off)
+    return c2 + b * c1;
+}
+// FP64 point: x[0..8] the own row at nu-4 .. nu+4, x[9..12] rows mu-1 .. mu-4,
+// x[13..16] rows mu+1 .. mu+4; am, ap: weights of the rows mu-+4 .. mu-+1;
+// c1, c2: d/dnu and d2/dnu2 weights at distance 4 .. 1.
+__device__ __forceinline__ double mcsor_point(const double *x, const double *am, const double *ap, const double *c1,
+                                              const double *c2, double dn, double lv, double rv, double om1)
+{
+#pragma clang fp contract(off)
+    const double d4 = fma_t(am[0], x[12], ap[0] * x[16]), d3 = fma_t(am[1], x[11], ap[1] * x[15]);
+    const double d2 = fma_t(am[2], x[10], ap[2] * x[14]), d1 = fma_t(am[3], x[9], ap[3] * x[13]);
+    const double dmu = (d4 + d3) + (d2 + d1);
+    const double ddni2 = fma_t(c2[0], x[0] + x[8], c2[1] * (x[1] + x[7])) +
+                         fma_t(c2[2], x[2] + x[6], c2[3] * (x[3] + x[5]));
+    const double ddni1 = fma_t(c1[0], x[0] - x[8], c1[1] * (x[1] - x[7])) +
+                         fma_t(c1[2], x[2] - x[6], c1[3] * (x[3] - x[5]));
+    const double cc = fma_t(dn, ddni1, dmu + ddni2);
+    return fma_t(rv - cc, lv, om1 * x[4]);
+}
+// Boundary value from the five next to it, nearest first: along nu, and along mu.
+template <typename T>
+__device__ __forceinline__ T mcsor_edge_nu(const T *ex, T v0, T v1, T v2, T v3, T v4)
+{
+#pragma clang fp contract(off)
+    return fma_t(ex[4], v4, fma_t(ex[3], v3, fma_t(ex[2], v2, fma_t(ex[0], v0, ex[1] * v1))));
+}
+template <typename T>
+__device__ __forceinline__ T mcsor_edge_mu(const T *ex, T v0, T v1, T v2, T v3, T v4)
+{
+#pragma clang fp contract(off)
+    return fma_t(ex[4], v4, fma_t(ex[3], v3, fma_t(ex[2], v2, fma_t(ex[1], v1, ex[0] * v0))));
+}
+
 // Kernel-level entry points shared between translation units.
 int launch_putin(x2g_grid *g, int isym, const double *fun, double *w1, double *w2);
 int launch_putout(x2g_grid *g, double *fun, const double *work);

@@ -1,0 +1,22 @@
+// Col-wise FP64 MCSOR of small grids, resident in LDS (x2gpu_resident.hip).
+#pragma once
+#include "x2gpu_internal.h"
+
+namespace x2g {
+
+struct ResidentDesc {
+    double *work;              // padded, row stride nni + 8; relaxed in place
+    const double *lr;          // (omega/lhs, rhs) pairs in the colour order of k_pack
+    const double *bmu, *dnu;
+    double c[16], ex[5], omega1;
+    int nni, nmu, even, per;   // per: threads of a row
+};
+// Whether a grid fits one compute unit.
+bool resident_fits(const x2g_ctx *ctx, int nni, int nmu);
+// Everything of a problem but its arrays.
+ResidentDesc resident_desc(const x2g_grid *g, int bkind, int isym, double omega);
+// nsweeps sweeps of every problem (each must fit).
+int launch_resident(x2g_ctx *ctx, std::vector<ResidentDesc> &v, int nsweeps);
+int resident_lds_attr(x2g_ctx *ctx);
+
+}  // namespace x2g

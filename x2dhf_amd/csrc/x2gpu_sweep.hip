@@ -29,6 +29,7 @@
 #include "x2gpu_internal.h"
 #include "x2gpu_chain.h"
 #include "x2gpu_front.h"
+#include "x2gpu_resident.h"
 #include <algorithm>
 #include <string>
 #include <atomic>
@@ -619,7 +620,7 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
     // Thread tid < 8 BR forms entry tid & 7 of row tid >> 3 of a block; its
     // two coefficients are loaded once.
     const T rw_c2 = d.c[4 + (tid & 3)], rw_c1 = d.c[tid & 3];
-    auto row_weight = [&](T b) -> T { return (tid & 7) < 4 ? rw_c2 + b * rw_c1 : rw_c2 - b * rw_c1; };
+    auto row_weight = [&](T b) -> T { return mcsor_row_weight((tid & 7) < 4 ? b : -b, rw_c1, rw_c2); };
 
     // the chunks of block bl, plus b(mu) of row (tid >> 3) % BR of the block
     // for the row weights (rows outside the grid read b = 0)
@@ -665,11 +666,8 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
                 const T *row = wbase + rr * W;
                 const int e1 = (cinfo[j] >> 3) & 7, e2 = (cinfo[j] >> 6) & 7;
                 const int c0 = nni + 3;
-                const T v1 = even ? d.ex[0] * row[5] + d.ex[1] * row[6] + d.ex[2] * row[7] + d.ex[3] * row[8] +
-                                        d.ex[4] * row[9]
-                                  : T(0);
-                const T v2 = even ? d.ex[0] * row[c0 - 1] + d.ex[1] * row[c0 - 2] + d.ex[2] * row[c0 - 3] +
-                                        d.ex[3] * row[c0 - 4] + d.ex[4] * row[c0 - 5]
+                const T v1 = even ? mcsor_edge_nu(d.ex, row[5], row[6], row[7], row[8], row[9]) : T(0);
+                const T v2 = even ? mcsor_edge_nu(d.ex, row[c0 - 1], row[c0 - 2], row[c0 - 3], row[c0 - 4], row[c0 - 5])
                                   : T(0);
 #pragma unroll
                 for (int k = 0; k < VEC; ++k) c.v[k] = k == e1 ? v1 : (k == e2 ? v2 : c.v[k]);
@@ -865,14 +863,8 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
                         T *w = okv[g][j] ? dnu_s + ov[g][j] + 4 : sink + tid;
                         *w = v;
                     } else {
-                        const T dmu = (am4 * xv[12] + ap4 * xv[16]) + (am3 * xv[11] + ap3 * xv[15]) +
-                                      ((am2 * xv[10] + ap2 * xv[14]) + (am1 * xv[9] + ap1 * xv[13]));
-                        const T ddni2 = (cf[4] * (xv[0] + xv[8]) + cf[5] * (xv[1] + xv[7])) +
-                                        (cf[6] * (xv[2] + xv[6]) + cf[7] * (xv[3] + xv[5]));
-                        const T ddni1 = (cf[0] * (xv[0] - xv[8]) + cf[1] * (xv[1] - xv[7])) +
-                                        (cf[2] * (xv[2] - xv[6]) + cf[3] * (xv[3] - xv[5]));
-                        const T cc = (dmu + ddni2) + dnu_s[cb] * ddni1;
-                        const T v = (rv[rr][j] - cc) * lv[rr][j] + om1 * xv[4];
+                        const T am[4] = {am4, am3, am2, am1}, ap[4] = {ap4, ap3, ap2, ap1};
+                        const T v = mcsor_point(xv, am, ap, cf, cf + 4, dnu_s[cb], lv[rr][j], rv[rr][j], om1);
                         T *w = okv[g][j] ? b0 + cb + rr * W + 4 : sink + tid;
                         *w = v;
                     }
@@ -906,11 +898,10 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
     auto row_one = [&]() {
         constexpr int RT = (W + 319) / 320;
         auto r1 = [&](int nu) -> T {
-            T acc = T(0);
+            T v[5];
 #pragma unroll
-            for (int k = 0; k < 5; ++k)
-                acc += d.ex[k] * buf_load1(rs_dst, (unsigned)(((5 + k) * P + nu + 3) * (int)sizeof(T)), T(0));
-            return acc;
+            for (int k = 0; k < 5; ++k) v[k] = buf_load1(rs_dst, (unsigned)(((5 + k) * P + nu + 3) * (int)sizeof(T)), T(0));
+            return mcsor_edge_mu(d.ex, v[0], v[1], v[2], v[3], v[4]);
         };
 #pragma unroll
         for (int k = 0; k < RT; ++k) {
@@ -921,8 +912,8 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
             if (even) {
                 if (nu == 1 || nu == nni) {
                     const int dir = nu == 1 ? 1 : -1;
-                    v = d.ex[0] * r1(nu + dir) + d.ex[1] * r1(nu + 2 * dir) + d.ex[2] * r1(nu + 3 * dir) +
-                        d.ex[3] * r1(nu + 4 * dir) + d.ex[4] * r1(nu + 5 * dir);
+                    v = mcsor_edge_nu(d.ex, r1(nu + dir), r1(nu + 2 * dir), r1(nu + 3 * dir), r1(nu + 4 * dir),
+                                      r1(nu + 5 * dir));
                 } else {
                     v = r1(nu);
                 }
@@ -1833,6 +1824,16 @@ static int sweep_kind(x2g_ctx *ctx, int maxnni)
     return choose_skew<T>(ctx, maxnni) > 0 ? 1 : 0;
 }
 
+// Kind 4: FP64 problems each resident on a compute unit, all sweeps in one
+// launch.  10 sweeps of 91 x 121 take 110 microseconds so and 313 with a
+// k_sweep launch each, whatever the number of problems up to the compute
+// units'.  Only where all problems of a batch are that small: among large
+// ones they cost a k_sweep launch next to nothing.
+static bool use_resident(x2g_ctx *ctx, int kind, int nni, int nmu)
+{
+    return kind == 2 && env_engine() == 0 && env_strip_l() <= 0 && !g_plan_fixed && resident_fits(ctx, nni, nmu);
+}
+
 // Launch one sweep of every problem in `descs` (device copy dd, host copy hv).
 // k_sweep for the plan's stride class and depth (the instantiations are
 // listed once here and in set_lds_attr).
@@ -1976,8 +1977,8 @@ static int set_lds_attr(x2g_ctx *ctx)
         (const void *)k_sweep<float, 1, 528, 2>,
         (const void *)k_sweep<float, 2, 768, 2>};
     for (const void *k : ks) X2G_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, mx));
-    const int rc = front_lds_attr(ctx);
-    if (rc) return rc;
+    int rc = front_lds_attr(ctx);
+    if (rc || (rc = resident_lds_attr(ctx))) return rc;
     done = true;
     return X2G_OK;
 }
@@ -2841,7 +2842,9 @@ static size_t mcsor_ws_bytes(const x2g_grid *g, int kind)
     const size_t ubytes = g->npad() * sizeof(double);
     const size_t pbytes = (size_t)P * (g->nmu + 8) * sizeof(double);
     const size_t lrbytes = 2 * split_size(g->nni, g->nmu) * sizeof(double);
-    return kind == 2 ? 2 * align256(pbytes) + align256(lrbytes) : align256(ubytes);
+    return kind == 4   ? align256(lrbytes)
+           : kind == 2 ? 2 * align256(pbytes) + align256(lrbytes)
+                       : align256(ubytes);
 }
 
 // mcsor of one padded array; the workspace is w0 (at least mcsor_ws_bytes).
@@ -2860,6 +2863,15 @@ static int mcsor_run(x2g_grid *g, int isym, int bkind, double *work_d, const dou
     const size_t lrbytes = 2 * split_size(g->nni, g->nmu) * sizeof(double);
     // k_sweep: two buffers of stride P and the (omega/lhs, rhs) pairs; the
     // other kinds: a ping-pong partner of the caller's array
+    if (kind == 4) {
+        double *lr = (double *)w0;
+        if ((rc = launch_pack<double>(ctx, {{lhs_d, lr, omega, g->nni, g->nmu, 0}, {rhs_d, lr, 0.0, g->nni, g->nmu, 1}})))
+            return rc;
+        std::vector<ResidentDesc> v{resident_desc(g, bkind, isym, omega)};
+        v[0].work = work_d;
+        v[0].lr = lr;
+        return launch_resident(ctx, v, nsweeps);
+    }
     const bool restride = kind == 2;
     double *A = work_d, *B = (double *)w0;
     if (restride) {
@@ -2914,7 +2926,8 @@ extern "C" int x2g_mcsor(x2g_grid *g, int isym, int bkind, double *work_d, const
     if (rc || nsweeps == 0) return rc;
     x2g_ctx *ctx = g->ctx;
     if ((rc = set_lds_attr(ctx))) return rc;
-    const int kind = sweep_kind<double>(ctx, g->nni);
+    int kind = sweep_kind<double>(ctx, g->nni);
+    if (use_resident(ctx, kind, g->nni, g->nmu)) kind = 4;
     if ((rc = ws_reserve(ctx, 0, mcsor_ws_bytes(g, kind)))) return rc;
     return mcsor_run(g, isym, bkind, work_d, lhs_d, rhs_d, omega, nsweeps, kind, (char *)ctx->ws[0].ptr);
 }
@@ -2927,7 +2940,8 @@ extern "C" int x2g_mcsor_noalloc(x2g_grid *g, int isym, int bkind, double *work_
     x2g_ctx *ctx = g->ctx;
     X2G_CHECK(ctx->scratch, "x2g_mcsor_noalloc: no scratch address for device %d", ctx->device);
     if ((rc = set_lds_attr(ctx))) return rc;
-    const int kind = sweep_kind<double>(ctx, g->nni);
+    int kind = sweep_kind<double>(ctx, g->nni);
+    if (use_resident(ctx, kind, g->nni, g->nmu)) kind = 4;
     const size_t need = mcsor_ws_bytes(g, kind);
     X2G_CHECK(need <= ctx->scratch_bytes,
               "x2g_mcsor_noalloc: grid %dx%d needs %zu bytes of scratch, more than its %zu (use x2g_mcsor)", g->nni,
@@ -3025,7 +3039,13 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
         if ((rc = check_grid_sweepable(g))) return rc;
         if (!ordered(it)) (it.prec ? maxnni32 : maxnni64) = std::max(it.prec ? maxnni32 : maxnni64, g->nni);
     }
-    const int kind64 = maxnni64 ? sweep_kind<double>(ctx, maxnni64) : 0;
+    int kind64 = maxnni64 ? sweep_kind<double>(ctx, maxnni64) : 0;
+    bool small = true;
+    for (int i = 0; i < n && small; ++i) {
+        const x2g_grid *g = grids[items[i].grid_index];
+        if (items[i].prec == 0 && !ordered(items[i])) small = use_resident(ctx, kind64, g->nni, g->nmu);
+    }
+    if (maxnni64 && small) kind64 = 4;
     int kind32 = maxnni32 ? sweep_kind<float>(ctx, maxnni32) : 0;
     // kind 3: the FP32 items, those of a grid and b(mu) together, as chains
     // where that is faster (and no engine or cut is asked for)
@@ -3123,7 +3143,7 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
         if (ordered(it))
             pin.push_back({it.fun_d, bufA(i), nullptr, g->nni, g->nmu, it.isym, g->nni + 8});
         else if (it.prec == 0)
-            pin.push_back({it.fun_d, bufA(i), bufB(i), g->nni, g->nmu, it.isym, pstride(i)});
+            pin.push_back({it.fun_d, bufA(i), kind64 == 4 ? nullptr : bufB(i), g->nni, g->nmu, it.isym, pstride(i)});
         if (it.tail_fock1_d)
             tails.push_back({it.fun_d, it.tail_fock1_d, g->suppl + 5 * g->n(), g->vxisq, g->vetasq, g->nni, g->nmu});
     }
@@ -3156,6 +3176,7 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
     // FP64 items: sweep plan
     SweepPlan<double> p64;
     const SweepDesc<double> *d64e = nullptr, *d64o = nullptr;
+    std::vector<ResidentDesc> res64;
     std::vector<PadDesc> pout64;
     if (!i64.empty()) {
         std::vector<SweepDesc<double>> base(i64.size());
@@ -3170,7 +3191,7 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
             base[k].lr = lrp(i64[k]);
             base[k].lr_bytes = (unsigned)lrbytes(i64[k]);
         }
-        if (kind64 == 2) {
+        if (kind64 == 2 || kind64 == 4) {
             // lhs / rhs do not change during the call: one residue-split copy
             std::vector<PackDesc<double>> pk;
             for (size_t k = 0; k < i64.size(); ++k) {
@@ -3181,11 +3202,20 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
             }
             if ((rc = launch_pack(ctx, pk))) return rc;
         }
-        SweepKnobs kn64;
-        if ((rc = tuned_knobs<double>(ctx, base, A, B, false, kn64))) return rc;
-        plan_sweeps(ctx, base, A, B, p64, &kn64);
-        if ((rc = stage_plan(ctx, p64, &d64e, &d64o))) return rc;
-        const bool final_in_b = p64.kind != 0 && (maxsor2 % 2) == 1;
+        if (kind64 == 4) {
+            for (size_t k = 0; k < i64.size(); ++k) {
+                const x2g_relax_item &it = items[i64[k]];
+                res64.push_back(resident_desc(grids[it.grid_index], it.bkind, it.isym, it.omega));
+                res64.back().work = A[k];
+                res64.back().lr = lrp(i64[k]);
+            }
+        } else {
+            SweepKnobs kn64;
+            if ((rc = tuned_knobs<double>(ctx, base, A, B, false, kn64))) return rc;
+            plan_sweeps(ctx, base, A, B, p64, &kn64);
+            if ((rc = stage_plan(ctx, p64, &d64e, &d64o))) return rc;
+        }
+        const bool final_in_b = kind64 != 4 && p64.kind != 0 && (maxsor2 % 2) == 1;
         for (size_t k = 0; k < i64.size(); ++k) {
             const x2g_relax_item &it = items[i64[k]];
             x2g_grid *g = grids[it.grid_index];
@@ -3361,7 +3391,8 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
             X2G_HIP(hipGetLastError());
         }
         if (!i64.empty()) {
-            if ((rc = launch_sweeps<double>(ctx, d64e, d64o, p64, maxsor2))) return rc;
+            rc = kind64 == 4 ? launch_resident(ctx, res64, maxsor2) : launch_sweeps<double>(ctx, d64e, d64o, p64, maxsor2);
+            if (rc) return rc;
             X2G_LAUNCH(ctx, k_putout, dim3(grid_x_for(maxn, 256), (int)i64.size()), dim3(256), 0,
                                d_pout64);
             X2G_HIP(hipGetLastError());

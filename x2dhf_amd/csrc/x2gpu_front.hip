@@ -49,7 +49,7 @@ struct FrontDesc {
     unsigned *done;                   // levels done of each sweep, kFlagGap apart
     double c[16], ex[5], omega, omega1;
     Strand st[2];
-    int nni, nmu, even, nst, ckind, cmid, ld, rows, last;   // last: step past the last block
+    int nni, nmu, even, nst, ckind, cmid, cmax, ld, rows, last;   // cmax: largest C; last: step past the last block
 };
 
 // Level of column nu.  The outer columns nu = 1, nni are extrapolated from
@@ -149,15 +149,24 @@ __global__ void __launch_bounds__(NT) k_front(const FrontDesc *__restrict__ fd, 
     // lanes past the halos do the last halo column's work again, unseen
     const int j0 = (wave - sn * per) * 64 + lane;
     const bool lane_on = on && j0 < ncol;
-    const int j = lane_on ? j0 : ncol - 1, nu = j - 3;
+    const unsigned j = lane_on ? j0 : ncol - 1;
+    const int nu = (int)j - 3;
     const bool inner = lane_on && nu >= 2 && nu <= nni - 1;
     const bool edge = lane_on && (nu == 1 || nu == nni);
     const bool any_edge = __any(edge);
     const int C = front_col(d.ckind, d.cmid, nni, nu);
     double *const ring = lds + (size_t)sn * kRingRows * W;
-    double *const tab = lds + (size_t)d.nst * kRingRows * W;  // b(mu), its sign the strand's way
-    double *const row1 = tab + nmu;                            // mu = 1, where the rows start there
-    for (int k = threadIdx.x; k < nmu; k += blockDim.x) tab[k] = d.bmu[k];
+    double *const row1 = lds + (size_t)d.nst * kRingRows * W;  // mu = 1, where the rows start there
+    // b(mu) of a strand's rows, its sign the strand's way, from level kFirst of
+    // the largest C on
+    const int tlo = d.cmax + kLevOff, tn = tlo + d.last;
+    double *const tabs = row1 + W;
+    for (int q = 0; q < d.nst; ++q)
+        for (int k = threadIdx.x; k < tn; k += blockDim.x) {
+            const int r = k - tlo, mu = d.st[q].mu0 + d.st[q].dir * r;
+            const double b = r >= 0 && r < d.st[q].len ? d.bmu[mu - 1] : 0.0;
+            tabs[q * tn + k] = d.st[q].dir > 0 ? b : -b;
+        }
     const double c0 = d.c[0], c1 = d.c[1], c2 = d.c[2], c3 = d.c[3], c4 = d.c[4], c5 = d.c[5], c6 = d.c[6],
                  c7 = d.c[7], c8 = d.c[8], c9 = d.c[9], c10 = d.c[10], c11 = d.c[11], c12 = d.c[12], c13 = d.c[13],
                  c14 = d.c[14], c15 = d.c[15];
@@ -165,17 +174,29 @@ __global__ void __launch_bounds__(NT) k_front(const FrontDesc *__restrict__ fd, 
     const double omega = d.omega, omega1 = d.omega1;
     const double dn = inner ? d.dnu[nu - 1] : 0.0;
     const bool even = d.even != 0;
-    const double sgn = st.dir > 0 ? 1.0 : -1.0;
     const bool up1 = st.dir > 0 && st.mu0 == 2;           // walks up from mu = 2: mu = 1 follows row 4
     const int r_mu1 = st.dir < 0 ? st.len - 1 : -100000;  // walks down to mu = 1
     const bool second = sn == 1;
     const int last = d.last, ld = d.ld;
     const size_t sbase = (size_t)sn * d.rows * ld;
-    double *const fsj = d.fs + sbase + j;                  // + (level + kLevOff) * ld
-    const double *const rsj = d.rs + sbase + j, *const lsj = d.ls + sbase + j;
+    double *const fsl = d.fs + sbase;                      // + (level + kLevOff) * ld + column
+    const double *const rsl = d.rs + sbase, *const lsl = d.ls + sbase;
+    const unsigned len_own = inner || edge ? (unsigned)st.len : 0u;   // rows this lane relaxes
     unsigned *const done = d.done + (size_t)sweep * kFlagGap;
     const unsigned *const before = done - kFlagGap;        // of the sweep before
     const int lev0 = st.lev0;
+    const double *const tab = tabs + sn * tn + tlo - C;
+    // levels of the wave's columns
+    int cmin = C, cmax = C;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        cmin = min(cmin, __shfl_xor(cmin, o, 64));
+        cmax = max(cmax, __shfl_xor(cmax, o, 64));
+    }
+    cmin = __builtin_amdgcn_readfirstlane(cmin);
+    cmax = __builtin_amdgcn_readfirstlane(cmax);
+    const unsigned W8 = (unsigned)W;
+    const unsigned nbj = min(max((int)j, 4), ncol - 5);   // halo columns read within the ring, to no effect
 
     // wait (first thread) until the sweep before has done `need` levels
     int known = sweep == 0 ? last : 0;
@@ -202,9 +223,9 @@ __global__ void __launch_bounds__(NT) k_front(const FrontDesc *__restrict__ fd, 
 #pragma unroll
     for (int k = 0; k < kU; ++k) {
         const int i = kFirst - lev0 + k + kLevOff;
-        nf[k] = on ? get_agent(fsj + (size_t)(i + kAhead) * ld) : 0.0;
-        nr[k] = on ? gmem(rsj)[(size_t)i * ld] : 0.0;
-        nl[k] = on ? gmem(lsj)[(size_t)i * ld] : 1.0;
+        nf[k] = on ? get_agent(fsl + (size_t)(i + kAhead) * ld + j) : 0.0;
+        nr[k] = on ? gmem(rsl + (size_t)i * ld)[j] : 0.0;
+        nl[k] = on ? gmem(lsl + (size_t)i * ld)[j] : 1.0;
     }
 
     for (int l0 = kFirst; l0 < last; l0 += kU) {
@@ -221,21 +242,22 @@ __global__ void __launch_bounds__(NT) k_front(const FrontDesc *__restrict__ fd, 
 #pragma unroll
             for (int k = 0; k < kU; ++k) {
                 const int i = l0 - lev0 + kU + k + kLevOff;
-                nf[k] = get_agent(fsj + (size_t)(i + kAhead) * ld);
-                nr[k] = gmem(rsj)[(size_t)i * ld];
-                nl[k] = gmem(lsj)[(size_t)i * ld];
+                nf[k] = get_agent(fsl + (size_t)(i + kAhead) * ld + j);
+                nr[k] = gmem(rsl + (size_t)i * ld)[j];
+                nl[k] = gmem(lsl + (size_t)i * ld)[j];
             }
         }
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
+            // (conditions on a whole wave first: they are scalar)
             const int lr = l0 + u - lev0, r = lr - C;
-            const bool act = lane_on && r >= 0 && r < st.len;
+            const int rmin = lr - cmax, rmax = lr - cmin;
             if (on) {
-                double *const own = ring + j;
-                double *const my = own + (r & (kRingRows - 1)) * W;
-                if (__any(act)) {
+                const unsigned slot = __umul24((unsigned)r & (kRingRows - 1), W8);
+                double *const my = ring + slot + j;
+                if (rmax >= 0 && rmin < st.len) {
                     double *const wp = w + 5 + u;
-                    if (second && __any(r == 0)) {
+                    if (second && rmin <= 0) {
                         // the rows below the first are the other strand's first four
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
@@ -243,11 +265,10 @@ __global__ void __launch_bounds__(NT) k_front(const FrontDesc *__restrict__ fd, 
                             if (r == 0) wp[-1 - k] = x;
                         }
                     }
-                    // halo columns read within the ring, to no effect
-                    const double *const nb = ring + (r & (kRingRows - 1)) * W + min(max(j, 4), ncol - 5);
+                    const double *const nb = ring + slot + nbj;
                     const double m4 = nb[-4], p4 = nb[4], m3 = nb[-3], p3 = nb[3], m2 = nb[-2], p2 = nb[2],
                                  m1 = nb[-1], p1 = nb[1];
-                    const double b = sgn * tab[min(max(st.mu0 + st.dir * r, 1), nmu) - 1];
+                    const double b = tab[lr];
                     const double ddmi2 = c4 * (wp[-4] + wp[4]) + c5 * (wp[-3] + wp[3]) + c6 * (wp[-2] + wp[2]) +
                                          c7 * (wp[-1] + wp[1]);
                     const double ddmi1 = c0 * (wp[-4] - wp[4]) + c1 * (wp[-3] - wp[3]) + c2 * (wp[-2] - wp[2]) +
@@ -256,7 +277,8 @@ __global__ void __launch_bounds__(NT) k_front(const FrontDesc *__restrict__ fd, 
                     const double ddni1 = c8 * (m4 - p4) + c9 * (m3 - p3) + c10 * (m2 - p2) + c11 * (m1 - p1);
                     const double cc = ddmi2 + b * ddmi1 + ddni2 + dn * ddni1;
                     double v = omega * (cr[u] - cc) / cl[u] + omega1 * wp[0];
-                    if (__any(inner && (r == r_mu1 || (up1 && r == 5)))) {
+                    double *const row = fsl + (size_t)(lr + kLevOff) * ld;   // the same for all lanes
+                    if ((rmin <= r_mu1 && rmax >= r_mu1) || (up1 && rmin <= 5 && rmax >= 5)) {
                         // mu = 1 from the five rows next to it
                         double x = 0.0;
                         if (even && up1)
@@ -266,31 +288,36 @@ __global__ void __launch_bounds__(NT) k_front(const FrontDesc *__restrict__ fd, 
                         if (r == r_mu1) v = x;
                         if (inner && up1 && r == 5) {
                             row1[j] = x;
-                            put_agent(fsj + (size_t)(lr - 6 + kLevOff) * ld, x);
+                            put_agent(row - (size_t)6 * ld + j, x);
                         }
                     }
-                    if (any_edge && edge) {
-                        const int to = nu == 1 ? 1 : -1;
-                        const double *const e = ring + (r & (kRingRows - 1)) * W + j;
-                        v = even ? ex0 * e[to] + ex1 * e[2 * to] + ex2 * e[3 * to] + ex3 * e[4 * to] + ex4 * e[5 * to]
-                                 : 0.0;
-                        if (up1 && r == 5) {
-                            const double *const o = row1 + j;
-                            put_agent(fsj + (size_t)(lr - 6 + kLevOff) * ld,
-                                      even ? ex0 * o[to] + ex1 * o[2 * to] + ex2 * o[3 * to] + ex3 * o[4 * to] +
-                                                 ex4 * o[5 * to]
-                                           : 0.0);
+                    if (any_edge) {
+                        if (edge) {
+                            const int to = nu == 1 ? 1 : -1;
+                            v = even ? ex0 * my[to] + ex1 * my[2 * to] + ex2 * my[3 * to] + ex3 * my[4 * to] +
+                                           ex4 * my[5 * to]
+                                     : 0.0;
+                            if (up1 && r == 5) {
+                                const double *const o = row1 + j;
+                                put_agent(row - (size_t)6 * ld + j,
+                                          even ? ex0 * o[to] + ex1 * o[2 * to] + ex2 * o[3 * to] + ex3 * o[4 * to] +
+                                                     ex4 * o[5 * to]
+                                               : 0.0);
+                            }
                         }
                     }
-                    if (act && (inner || edge)) {
+                    if (((unsigned)r < len_own)) {
                         wp[0] = v;
                         *my = v;
-                        put_agent(fsj + (size_t)(lr + kLevOff) * ld, v);
-                        // the first rows of the second strand lie behind row 0 of the first
-                        if (second && r < 4) put_agent(d.fs + (size_t)(C - 1 - r + kLevOff) * ld + j, v);
+                        put_agent(row + j, v);
+                    }
+                    // the first rows of the second strand lie behind row 0 of the first
+                    if (second && rmin < 4) {
+                        if ((unsigned)r < min(len_own, 4u))
+                            put_agent(d.fs + (size_t)(C - 1 - r + kLevOff) * ld + j, v);
                     }
                 }
-                if (lane_on) own[((r + kAhead) & (kRingRows - 1)) * W] = w[5 + u + kAhead];
+                if (lane_on) ring[__umul24(((unsigned)r + kAhead) & (kRingRows - 1), W8) + j] = w[5 + u + kAhead];
             }
             if (u == kU - 1) {
                 // this wave's stores are at the agent's coherence point
@@ -336,36 +363,17 @@ static bool front_ways(int method, int ordering, int &rows, int &cols)
 }
 
 static int front_threads(int nni, int nst) { return ((nni + 8 + 63) & ~63) * nst; }
-static size_t front_lds(int nni, int nmu, int nst)
+static size_t front_lds(const FrontDesc &d)
 {
-    const size_t W = (nni + 8 + 31) & ~31;
-    return ((size_t)nst * kRingRows * W + nmu + W) * sizeof(double);
+    const size_t W = (d.nni + 8 + 31) & ~31;
+    return ((size_t)d.nst * kRingRows * W + W + (size_t)d.nst * (d.cmax + kLevOff + d.last)) * sizeof(double);
 }
 
-bool front_fits(const x2g_ctx *ctx, int nni, int nmu, int method, int ordering)
+// Strands, levels and sizes of a grid in one order.
+static FrontDesc front_shape(int nni, int nmu, int method, int ordering)
 {
-    int rows, cols;
-    if (!front_ways(method, ordering, rows, cols)) return false;
-    const int nst = rows == kMirrored ? 2 : 1;
-    return nni >= kMinFront && nmu >= kMinFront && (long)nmu * nni < (1L << 28) && front_threads(nni, nst) <= 1024 &&
-           front_lds(nni, nmu, nst) + 64 <= ctx->max_lds;
-}
-
-int front_lds_attr(x2g_ctx *ctx)
-{
-    const int lds = (int)ctx->max_lds - 64;   // the static part is one word
-    X2G_HIP(hipFuncSetAttribute((const void *)k_front<512>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    X2G_HIP(hipFuncSetAttribute((const void *)k_front<768>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    X2G_HIP(hipFuncSetAttribute((const void *)k_front<1024>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    return X2G_OK;
-}
-
-// Strands, levels and sizes of an item.
-static FrontDesc front_shape(const FrontItem &it)
-{
-    const int nni = it.g->nni, nmu = it.g->nmu;
     int rw = kStraight, cw = kStraight;
-    front_ways(it.method, it.ordering, rw, cw);
+    front_ways(method, ordering, rw, cw);
     FrontDesc d{};
     d.nni = nni;
     d.nmu = nmu;
@@ -381,15 +389,36 @@ static FrontDesc front_shape(const FrontItem &it)
         d.st[0] = {mid, -1, mid, 0};
         d.st[1] = {mid + 1, 1, nmu - 4 - mid, 4};
     }
-    int cmax = 0, steps = 0;
-    for (int nu = 1; nu <= nni; ++nu) cmax = std::max(cmax, front_col(cw, d.cmid, nni, nu));
+    // (the outer columns come after those next to them)
+    const int cmax = std::max(front_col(cw, d.cmid, nni, 1), front_col(cw, d.cmid, nni, nni));
+    int steps = 0;
     for (int s = 0; s < d.nst; ++s) steps = std::max(steps, d.st[s].lev0 + d.st[s].len + cmax);
     steps -= kFirst;
+    d.cmax = cmax;
     d.last = kFirst + (steps + kU - 1) / kU * kU;
     d.ld = (nni + 8 + 7) & ~7;
     d.rows = d.last + kU + kAhead + kLevOff;   // the last block's loads end there
     return d;
 }
+
+bool front_fits(const x2g_ctx *ctx, int nni, int nmu, int method, int ordering)
+{
+    int rows, cols;
+    if (!front_ways(method, ordering, rows, cols)) return false;
+    const int nst = rows == kMirrored ? 2 : 1;
+    return nni >= kMinFront && nmu >= kMinFront && (long)nmu * nni < (1L << 28) && front_threads(nni, nst) <= 1024 &&
+           front_lds(front_shape(nni, nmu, method, ordering)) + 64 <= ctx->max_lds;
+}
+
+int front_lds_attr(x2g_ctx *ctx)
+{
+    const int lds = (int)ctx->max_lds - 64;   // the static part is one word
+    X2G_HIP(hipFuncSetAttribute((const void *)k_front<512>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    X2G_HIP(hipFuncSetAttribute((const void *)k_front<768>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    X2G_HIP(hipFuncSetAttribute((const void *)k_front<1024>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    return X2G_OK;
+}
+
 static size_t front_array(const FrontDesc &d) { return (size_t)d.nst * d.rows * d.ld; }
 static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 static size_t front_bytes(const FrontDesc &d, int nsweeps)
@@ -400,7 +429,7 @@ static size_t front_bytes(const FrontDesc &d, int nsweeps)
 int front_reserve(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps)
 {
     size_t off = 256;   // the tickets first
-    for (auto &it : items) off += front_bytes(front_shape(it), nsweeps);
+    for (auto &it : items) off += front_bytes(front_shape(it.g->nni, it.g->nmu, it.method, it.ordering), nsweeps);
     // (a capture cannot allocate)
     if (ctx->cap_arena && ctx->ws[6].bytes < off) return X2G_ENOMEM;
     return ws_reserve(ctx, 6, off);
@@ -418,7 +447,7 @@ int launch_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps
     char *base = (char *)ctx->ws[6].ptr;
     for (auto &it : items) {
         const x2g_grid *g = it.g;
-        FrontDesc d = front_shape(it);
+        FrontDesc d = front_shape(g->nni, g->nmu, it.method, it.ordering);
         d.f = it.work;
         d.lhs = it.lhs;
         d.rhs = it.rhs;
@@ -436,7 +465,7 @@ int launch_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps
         d.done = (unsigned *)(base + off + align256(3 * n * sizeof(double)));
         off += front_bytes(d, nsweeps);
         nt = std::max(nt, front_threads(d.nni, d.nst));
-        lds = std::max(lds, front_lds(d.nni, d.nmu, d.nst));
+        lds = std::max(lds, front_lds(d));
         most = std::max(most, (int)n);
         bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5) * nsweeps;
         v.push_back(d);

@@ -474,7 +474,15 @@ __host__ __device__ inline size_t sweep_lds_elems(int W, int nth, int BR)
 template <typename T>
 constexpr int sweep_vec() { return 16 / (int)sizeof(T); }
 template <typename T>
-constexpr int sweep_nsv(int BR) { return sizeof(T) == 4 ? (BR == 4 ? 2 : 1) : (BR == 4 ? 3 : 2); }
+constexpr int sweep_nsv(int BR) { return sizeof(T) == 4 ? (BR == 4 ? 2 : 1) : 2; }
+// Waves that share a pass, each with its part of the rows of a block.  FP64
+// rings leave room for one workgroup on a CU, whose step is the length of a
+// pass wave's instructions: with two waves a pass (of two rows each, read
+// together as before) 10 sweeps of 22 potentials of 331 x 601 take 692
+// microseconds, with one 767.  FP32 runs two workgroups side by side, and
+// two-row blocks have no second pair of rows.
+template <typename T>
+__host__ __device__ constexpr int sweep_split(int BR) { return sizeof(T) == 8 && BR == 4 ? 2 : 1; }
 // row stride of k_sweep's padded arrays: nni+8 rounded up to 16 bytes
 __host__ __device__ inline int sweep_row_stride(int nni, int vec) { return (nni + 8 + vec - 1) / vec * vec; }
 
@@ -546,11 +554,12 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
 template <typename T, int W, int BR>
 constexpr int sweep_waves_per_eu()
 {
-    return sizeof(T) != 4 ? 1 : (BR == 4 ? (W <= 384 ? 4 : 1) : (W <= 256 ? 5 : (W <= 528 ? 4 : 1)));
+    return sizeof(T) != 4 ? (BR == 4 ? 3 : 1) : (BR == 4 ? (W <= 384 ? 4 : 1) : (W <= 256 ? 5 : (W <= 528 ? 4 : 1)));
 }
 
 template <typename T, int NT, int W, int BR>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sweep_waves_per_eu<T, W, BR>())))
+__global__ void __launch_bounds__(sweep_split<T>(BR) == 1 ? 512 : 768)
+    __attribute__((amdgpu_waves_per_eu(sweep_waves_per_eu<T, W, BR>())))
 k_sweep(const SweepDesc<T> *__restrict__ descs, const SweepSeg *__restrict__ segs, const int *__restrict__ wg_seg,
         int MS, int zero_src)
 {
@@ -576,6 +585,7 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
     // live window s-4 SKEW-R .. s+R plus the block being prefetched)
     constexpr int R = 4 / BR, SKEW = sweep_skew(BR), RB = sweep_ring_blocks(BR), RROWS = RB * BR;
     constexpr int VEC = sweep_vec<T>(), NSV = sweep_nsv<T>(BR);
+    constexpr int H = sweep_split<T>(BR), HR = BR / H;   // waves of a pass, rows of each
     T *const dnu_s = reinterpret_cast<T *>(ks_smem);
 
     const int nni = d.nni, nmu = d.nmu, P = d.P;
@@ -698,8 +708,10 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
     // row accepts, and toff = its byte offset in a row of (omega/lhs, rhs)
     // pairs, or kOOBLane for an absent point.
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const bool pass_wave = wave < 5;
-    const int q = tid - 320;
+    const bool pass_wave = wave < 5 * H;
+    const int spill = (5 * MS + 63) / 64 * 64;   // spill lanes of each part of the rows
+    const int part = H == 1 ? 0 : pass_wave ? wave / 5 : __builtin_amdgcn_readfirstlane(tid - 320 * H >= spill ? 1 : 0);
+    const int q = tid - 320 * H - (pass_wave ? 0 : part * spill);
     const int MSp = max(0, min(MS, M - 64 * NT));
     const int p_spill = pass_wave || q >= 5 * MSp ? 5 : q / MSp;
     constexpr int kNoPoint = 1 << 20;
@@ -723,12 +735,12 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
     // (omega/lhs, rhs) of pass p's points in step s (rows of block
     // s - SKEW p); rows outside the pass's range or the grid and absent points
     // read zeros, which are never used
-    auto load_lr = [&](int s, int p, T (&lv)[BR][NT], T (&rv)[BR][NT]) {
+    auto load_lr = [&](int s, int p, T (&lv)[HR][NT], T (&rv)[HR][NT]) {
         const int b = s - SKEW * p;
         const bool act = p < 5 && b >= R * p && b <= K - 1 - R * p;
-        const int mu0 = r0 + BR * b;
+        const int mu0 = r0 + BR * b + HR * part;
 #pragma unroll
-        for (int rr = 0; rr < BR; ++rr) {
+        for (int rr = 0; rr < HR; ++rr) {
             const int mu = mu0 + rr;
             const bool rowok = act && mu >= 2 && mu <= nmu - 4;
             const unsigned rb = rowok ? (unsigned)(((mu - 2) * M5 + p * M) * (int)(2 * sizeof(T))) : kOOB;
@@ -755,8 +767,9 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
     // of one pass in a row do not read each other (a point's neighbours have
     // other colours), so a row's stencil values are gathered first and its
     // arithmetic follows, which keeps the LDS reads in flight together.
-    auto compute_rows = [&](int b, int p, const T (&lv)[BR][NT], const T (&rv)[BR][NT], auto contig) {
+    auto compute_rows = [&](int b, int p, const T (&lv)[HR][NT], const T (&rv)[HR][NT], auto contig, auto partc) {
         constexpr bool CONTIG = decltype(contig)::value;
+        constexpr int RR0 = decltype(partc)::value * HR;   // the first of its rows
         const int sb = slot_of(b);
         const T *const wb = ring + slot_of(b - R) * BR * W;  // the window's first block (CONTIG)
         // the ring blocks b-R .. b+R
@@ -770,20 +783,20 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
         T *const b0 = ring + sb * BR * W;         // block b
         const int mu0 = r0 + BR * b;
         const T *ab = ab_r + sb * 8 * BR;        // row weights of block b
-        int off = mod5(p - cA * (mu0 - 2));     // (nu-2) mod 5 of the pass's points in row mu0
+        int off = mod5(p - cA * (mu0 + RR0 - 2));     // (nu-2) mod 5 of the pass's points in its first row
         // Rows are processed in groups of G: the stencil values of a group are
         // gathered before its arithmetic (the points of one pass never read
         // each other, in one row or in neighbouring rows).
         constexpr int G = 2;
 #pragma unroll
-        for (int rg = 0; rg < BR; rg += G) {
+        for (int rg = RR0; rg < RR0 + HR; rg += G) {
             int cbv[G][NT], ov[G][NT];
             bool okv[G][NT];
             T x[G][NT][17];  // 0..8: own row at nu-4..nu+4; 9..12: rows mu-1..mu-4; 13..16: rows mu+1..mu+4
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const int rr = rg + g;
-                if (rr) off = off - cA < 0 ? off - cA + 5 : off - cA;
+                if (rr > RR0) off = off - cA < 0 ? off - cA + 5 : off - cA;
                 const int mu = mu0 + rr;
                 const int lim_r = mu >= 2 && mu <= nmu - 4 ? nni - 3 - off : -1;  // point ok iff 5t <= lim_r
 #pragma unroll
@@ -859,12 +872,12 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
                         t = __builtin_fmaf(cf[2], xv[2] - xv[6], t);
                         t = __builtin_fmaf(cf[3], xv[3] - xv[5], t);
                         acc = __builtin_fmaf(dnu_s[cb], t, acc);
-                        const float v = __builtin_fmaf(rv[rr][j] - acc, lv[rr][j], om1 * xv[4]);
+                        const float v = __builtin_fmaf(rv[rr - RR0][j] - acc, lv[rr - RR0][j], om1 * xv[4]);
                         T *w = okv[g][j] ? dnu_s + ov[g][j] + 4 : sink + tid;
                         *w = v;
                     } else {
                         const T am[4] = {am4, am3, am2, am1}, ap[4] = {ap4, ap3, ap2, ap1};
-                        const T v = mcsor_point(xv, am, ap, cf, cf + 4, dnu_s[cb], lv[rr][j], rv[rr][j], om1);
+                        const T v = mcsor_point(xv, am, ap, cf, cf + 4, dnu_s[cb], lv[rr - RR0][j], rv[rr - RR0][j], om1);
                         T *w = okv[g][j] ? b0 + cb + rr * W + 4 : sink + tid;
                         *w = v;
                     }
@@ -878,17 +891,17 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
     // scalar) whose window does not wrap reads all 17 stencil values of a
     // point from one base register with immediate offsets (FP32); otherwise
     // each block has its own base.
-    auto compute = [&](int s, int p, const T (&lv)[BR][NT], const T (&rv)[BR][NT], auto role) {
+    auto compute = [&](int s, int p, const T (&lv)[HR][NT], const T (&rv)[HR][NT], auto role, auto partc) {
         const int b = s - SKEW * p;
         if (p >= 5 || b < R * p || b > K - 1 - R * p) return;  // idle lanes and passes outside their range
         const int sw = slot_of(b - R);
         if constexpr (decltype(role)::value && sizeof(T) == 4) {
             if (sw + 2 * R < RB) {
-                compute_rows(b, p, lv, rv, std::true_type{});
+                compute_rows(b, p, lv, rv, std::true_type{}, partc);
                 return;
             }
         }
-        compute_rows(b, p, lv, rv, std::false_type{});
+        compute_rows(b, p, lv, rv, std::false_type{}, partc);
     };
     // The mu=1 row (sormcsor.F90:333-350) of the first strip, after its last
     // step: rows 2..6 are final in dst, written by this workgroup (the
@@ -935,22 +948,22 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
     // The two lane roles run separate copies of the step loop (each wave is
     // wholly in one role and every copy meets the same barriers), so that in
     // a pass wave the pass and all that depends on it stay scalar.
-    auto steps = [&](auto role) {
+    auto steps = [&](auto role, auto partc) {
         constexpr bool PASS = decltype(role)::value;
-        const int p = PASS ? wave : p_spill;
+        const int p = PASS ? wave - 5 * part : p_spill;
         const bool busy = PASS || !spill_idle;
-        T lv[BR][NT], rv[BR][NT];
+        T lv[HR][NT], rv[HR][NT];
         load_lr(0, p, lv, rv);
         for (int s = 0; s < S; ++s) {
-            T ln[BR][NT], rn[BR][NT], bpre;
+            T ln[HR][NT], rn[HR][NT], bpre;
             u32x4 pre[NSV];
             load_lr(s + 1, p, ln, rn);
             load_block(s + R + 1, pre, bpre);
             if (early_out) write_out(s - 4 * SKEW - R);
-            if (busy) compute(s, p, lv, rv, role);
+            if (busy) compute(s, p, lv, rv, role, partc);
             commit_block(s + R + 1, pre, bpre);
 #pragma unroll
-            for (int rr = 0; rr < BR; ++rr)
+            for (int rr = 0; rr < HR; ++rr)
 #pragma unroll
                 for (int j = 0; j < NT; ++j) {
                     lv[rr][j] = ln[rr][j];
@@ -960,8 +973,15 @@ __device__ __forceinline__ void sweep_segment(const SweepDesc<T> &d, const int a
             __syncthreads();
         }
     };
-    if (pass_wave) steps(std::true_type{});
-    else steps(std::false_type{});
+    constexpr std::integral_constant<int, 0> first{};
+    constexpr std::integral_constant<int, H - 1> second{};
+    if (H == 1 || part == 0) {
+        if (pass_wave) steps(std::true_type{}, first);
+        else steps(std::false_type{}, first);
+    } else {
+        if (pass_wave) steps(std::true_type{}, second);
+        else steps(std::false_type{}, second);
+    }
     if (a == 2) {
         __syncthreads();
         row_one();
@@ -1791,22 +1811,24 @@ static int sweep_stride(int maxnni)
 
 // Lanes of a k_sweep launch for a batch whose widest grid has nni points:
 // five pass waves with NT colour points per lane and row (64 NT per pass),
-// plus spill waves for the MS remaining points of each pass, one per lane.
-static void sweep_lanes(int maxnni, int &MS, int &NT, int &nth)
+// plus spill waves for the MS remaining points of each pass, one per lane;
+// `split` times (sweep_split).
+static void sweep_lanes(int maxnni, int split, int &MS, int &NT, int &nth)
 {
     const int M = split_m(maxnni);
     NT = M <= 102 ? 1 : 2;
     MS = std::max(0, M - 64 * NT);
-    nth = 320 + 64 * ((5 * MS + 63) / 64);
+    nth = split * (320 + 64 * ((5 * MS + 63) / 64));
 }
 
 template <typename T>
 static bool sweep_fits(x2g_ctx *ctx, int maxnni)
 {
     int MS, NT, nth;
-    sweep_lanes(maxnni, MS, NT, nth);
+    const int split = sweep_split<T>(4);
+    sweep_lanes(maxnni, split, MS, NT, nth);
     const int W = sweep_stride<T>(maxnni);
-    if (W == 0 || nth > 512 || (NT == 2) != (W == 768)) return false;
+    if (W == 0 || nth > (split == 1 ? 512 : 768) || (NT == 2) != (W == 768)) return false;
     // a block's 16-byte chunks must fit the threads' copy slots
     const int P = sweep_row_stride(maxnni, sweep_vec<T>());
     if (4 * P / sweep_vec<T>() > sweep_nsv<T>(4) * nth || P > W) return false;
@@ -2065,9 +2087,9 @@ static int plan_sweeps(x2g_ctx *ctx, std::vector<SweepDesc<T>> &base, std::vecto
                 cmax = std::max(cmax, base[i].nni);
                 rows.push_back(prow[i]);
             }
-            sweep_lanes(cmax, sub.MS, sub.NT, sub.nth);
             sub.W = kv.first;
             sub.br = (kn ? kn->br : g_sweep_br) == 2 ? 2 : 4;
+            sweep_lanes(cmax, sweep_split<T>(sub.br), sub.MS, sub.NT, sub.nth);
             sub.lds = sweep_lds_elems(sub.W, sub.nth, sub.br) * sizeof(T);
             int wpc = kn ? kn->wpc : g_sweep_wpc;
             if (wpc <= 0) wpc = std::max<int>(1, (int)(ctx->max_lds / std::max<size_t>(sub.lds, 1)));

@@ -90,12 +90,17 @@ static std::vector<ChainClass> chain_classes(const std::vector<ChainProblem> &pr
 
 // Choose the sweeps per launch and the steps of a workgroup: workgroups of
 // equal length that fill the chip as few times as it takes, or once more.
-// Returns the time.
-static double chain_cut(x2g_ctx *ctx, std::vector<ChainClass> &cls, int nsweeps, ChainCut &cut)
+// Only cuts of less than `limit` microseconds count, so that a call which is
+// better off without chains pays little for the question.  Returns the time
+// (limit: no cut).
+static double chain_cut(x2g_ctx *ctx, std::vector<ChainClass> &cls, int nsweeps, double limit, ChainCut &cut)
 {
-    double best = 1e300;
+    double best = limit;
     for (int sw = 1; sw <= kChainWaves && sw <= nsweeps; ++sw) {
         if (sw > 1 && (nsweeps + sw - 1) / sw == (nsweeps + sw - 2) / (sw - 1)) continue;   // as many launches
+        // the shortest segments there are: a whole grid's 56 rows, or one row with its halos
+        const int least = std::min(83 + 23 * (sw - 1), 43 + 43 * (sw - 1));
+        if ((nsweeps + sw - 1) / sw * (least * kStepTime + kLaunchTime) >= best) continue;
         bool ok = true;
         for (auto &c : cls) ok = ok && c.pack(sw);
         if (!ok) break;
@@ -113,7 +118,10 @@ static double chain_cut(x2g_ctx *ctx, std::vector<ChainClass> &cls, int nsweeps,
         const long whole = wgs(longest);
         const int r0 = (int)((whole + ctx->num_cu - 1) / ctx->num_cu);
         for (int rounds = r0; rounds < r0 + 2; ++rounds) {
-            int lo = 1, hi = longest;   // least steps with workgroups of `rounds` rounds
+            // least steps with workgroups of `rounds` rounds, where that is a better cut
+            const double room = (best / nch - kLaunchTime) / (rounds * kStepTime);
+            int lo = 1, hi = (int)std::min<double>(longest, room);
+            if (hi < least || wgs(hi) > (long)rounds * ctx->num_cu) continue;
             while (lo < hi) {
                 const int mid = (lo + hi) / 2;
                 if (wgs(mid) <= (long)rounds * ctx->num_cu) hi = mid;
@@ -143,7 +151,8 @@ bool chain_pays(x2g_ctx *ctx, const std::vector<ChainProblem> &probs, int nsweep
     }
     std::vector<ChainClass> cls = chain_classes(probs);
     // (less the estimates' errors)
-    return 1.08 * chain_cut(ctx, cls, nsweeps, cut) < nsweeps * t;
+    const double limit = nsweeps * t / 1.08;
+    return chain_cut(ctx, cls, nsweeps, limit, cut) < limit;
 }
 
 int chain_plan(x2g_ctx *ctx, const std::vector<ChainProblem> &probs, int nsweeps, const ChainCut &cut, ChainPlan &plan)

@@ -431,8 +431,8 @@ int front_reserve(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps
     size_t off = 256;   // the tickets first
     for (auto &it : items) off += front_bytes(front_shape(it.g->nni, it.g->nmu, it.method, it.ordering), nsweeps);
     // (a capture cannot allocate)
-    if (ctx->cap_arena && ctx->ws[6].bytes < off) return X2G_ENOMEM;
-    return ws_reserve(ctx, 6, off);
+    if (ctx->cap_arena && ctx->ws[4].bytes < off) return X2G_ENOMEM;
+    return ws_reserve(ctx, 4, off);
 }
 
 int launch_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps)
@@ -444,7 +444,7 @@ int launch_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps
     int nt = 0, most = 0;
     size_t lds = 0;
     double bytes = 0;
-    char *base = (char *)ctx->ws[6].ptr;
+    char *base = (char *)ctx->ws[4].ptr;
     for (auto &it : items) {
         const x2g_grid *g = it.g;
         FrontDesc d = front_shape(g->nni, g->nmu, it.method, it.ordering);
@@ -470,7 +470,7 @@ int launch_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps
         bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5) * nsweeps;
         v.push_back(d);
     }
-    X2G_CHECK(ctx->ws[6].bytes >= off, "launch_fronts: workspace");
+    X2G_CHECK(ctx->ws[4].bytes >= off, "launch_fronts: workspace");
     unsigned *tickets = (unsigned *)base;
     const FrontDesc *dd;
     if ((rc = stage_n(ctx, v.data(), v.size(), &dd)) || (rc = stage_flush(ctx))) return rc;

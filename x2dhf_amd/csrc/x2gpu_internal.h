@@ -45,11 +45,10 @@ struct x2g_ctx {
     hipStream_t stream = nullptr;
     int num_cu = 0;
     size_t max_lds = 0;
-    x2g::Workspace ws[7];          // 0: padded work buffers, 1: reduction partials,
+    x2g::Workspace ws[6];          // 0: padded work buffers, 1: reduction partials,
                                    // 2: launch descriptors, 3: FP32 staging,
-                                   // 4: padded buffers of batched quadratures,
-                                   // 5: batched reduction partials,
-                                   // 6: arrays by level of ordered sweeps
+                                   // 4: arrays by level of ordered sweeps,
+                                   // 5: batched reduction partials
     void *pinned = nullptr;        // pinned host staging for descriptors/results
     size_t pinned_bytes = 0;
     void *pinned_out = nullptr;    // pinned host buffer for gathered results
@@ -81,7 +80,7 @@ struct x2g_ctx {
     struct GraphEntry {
         hipGraphExec_t exec = nullptr;
         void *arena = nullptr;
-        void *ws0 = nullptr, *ws3 = nullptr, *ws6 = nullptr;  // workspace the graph addresses
+        void *ws0 = nullptr, *ws3 = nullptr, *ws4 = nullptr;  // workspace the graph addresses
         long last_use = 0;
     };
     bool graphs_on = false;
@@ -216,13 +215,6 @@ __device__ __forceinline__ T mcsor_edge_mu(const T *ex, T v0, T v1, T v2, T v3, 
 // Kernel-level entry points shared between translation units.
 int launch_putin(x2g_grid *g, int isym, const double *fun, double *w1, double *w2);
 int launch_putout(x2g_grid *g, double *fun, const double *work);
-// putin of several functions (each on its own grid) in one launch
-struct PadItem {
-    const double *fun;
-    double *w;
-    int nni, nmu, isym;
-};
-int launch_putin_items(x2g_ctx *ctx, const std::vector<PadItem> &items);
 // pinned host buffer of at least `bytes` for device -> host results
 int pinned_out_reserve(x2g_ctx *ctx, size_t bytes);
 // Look up the device address of the no-allocation scratch array on the

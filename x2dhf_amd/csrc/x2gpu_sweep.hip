@@ -1563,23 +1563,6 @@ int launch_putin(x2g_grid *g, int isym, const double *fun, double *w1, double *w
     return X2G_OK;
 }
 
-int launch_putin_items(x2g_ctx *ctx, const std::vector<PadItem> &items)
-{
-    if (items.empty()) return X2G_OK;
-    std::vector<PadDesc> v;
-    long maxpad = 0;
-    for (auto &it : items) {
-        v.push_back({it.fun, it.w, nullptr, it.nni, it.nmu, it.isym, it.nni + 8});
-        maxpad = std::max<long>(maxpad, (long)(it.nni + 8) * (it.nmu + 8));
-    }
-    const PadDesc *dd;
-    int rc = stage_n(ctx, v.data(), v.size(), &dd);
-    if (rc) return rc;
-    X2G_LAUNCH(ctx, k_putin, dim3(grid_x_for(maxpad, 256), (int)v.size()), dim3(256), 0, dd);
-    X2G_HIP(hipGetLastError());
-    return X2G_OK;
-}
-
 int launch_putout(x2g_grid *g, double *fun, const double *work)
 {
     std::vector<PadDesc> v{{fun, const_cast<double *>(work), nullptr, g->nni, g->nmu, 1, g->nni + 8}};
@@ -3478,7 +3461,7 @@ static std::string relax_signature(x2g_ctx *ctx, x2g_grid *const *grids, const x
     put(g_plan_gen.load());
     put(ctx->ws[0].ptr);
     put(ctx->ws[3].ptr);
-    put(ctx->ws[6].ptr);
+    put(ctx->ws[4].ptr);
     for (int i = 0; i < n; ++i) {
         const x2g_relax_item &it = items[i];
         const x2g_grid *g = grids[it.grid_index];
@@ -3567,7 +3550,7 @@ static int relax_capture(x2g_ctx *ctx, const std::string &key, x2g_grid *const *
         g.arena = arena;
         g.ws0 = ctx->ws[0].ptr;
         g.ws3 = ctx->ws[3].ptr;
-        g.ws6 = ctx->ws[6].ptr;
+        g.ws4 = ctx->ws[4].ptr;
         ++ctx->graph_captures;
         *out = &g;
         return X2G_OK;

@@ -83,6 +83,12 @@ int x2g_stats_enable(x2g_ctx *ctx, int on);
  * 4 words (read u, write u, read lhs, read rhs). */
 int x2g_stats_get(x2g_ctx *ctx, double *out);
 
+/* What the calls on this context did so far, out[X2G_COUNT_*] for the first n
+ * counts (those past the last are 0): bytes of launch descriptors staged. */
+#define X2G_COUNT_STAGED 0
+#define X2G_COUNTS 1
+int x2g_call_counts(x2g_ctx *ctx, long long *out, int n);
+
 /* ---- device memory ------------------------------------------------------ */
 /* Blocks freed with x2g_free stay with the context and are handed out again
  * by x2g_malloc for the same size (no synchronisation: all work of a

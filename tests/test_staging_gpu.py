@@ -1,0 +1,65 @@
+"""Launch descriptors of a relaxation call: what a call stages depends on its
+items, not on how often or how long they are relaxed, and every descriptor
+stays what it was until the call's last launch has read it.
+"""
+import numpy as np
+import pytest
+
+from oracle import pyoracle
+from test_kernels_gpu import synthetic_problem
+
+pytestmark = pytest.mark.gpu
+
+STAGED = 0  # X2G_COUNT_STAGED
+
+
+class Batch:
+    """count functions of one grid as relax items of one scheme."""
+
+    def __init__(self, ctx, nni, nmu, count, prec=0, method=0, ordering=0, seed=5):
+        from x2dhf_amd import gpu
+        self.ctx, self.P = ctx, synthetic_problem(nni, nmu, seed=seed)
+        P = self.P
+        self.grid = gpu.Grid(ctx, nni, nmu, P["coef"], P["suppl"], P["vxi"], P["veta"])
+        self.lhs, self.rhs = ctx.upload(P["lhs"]), ctx.upload(P["rhs"])
+        self.u = np.tile(P["fun"], (count, 1)) * (1.0 + 0.1 * (np.arange(count) % 5))[:, None]
+        self.f = ctx.upload(self.u)
+        items = []
+        for k in range(count):
+            it = gpu.RelaxItem(self.f.ptr + 8 * k * nni * nmu, self.lhs.ptr, self.rhs.ptr, None, 1.8, 1, 1, prec, 0)
+            it.method, it.ordering = method, ordering
+            items.append(it)
+        self.arr, self.n = (gpu.RelaxItem * count)(*items), count
+        self.gh = (gpu._vp * 1)(self.grid.h.value)
+
+    def relax(self, maxsor1, maxsor2):
+        """Bytes staged by one call from the starting functions; the results."""
+        from x2dhf_amd import gpu
+        self.f.set(self.u)
+        before = self.ctx.counts()[STAGED]
+        gpu.check(self.ctx.lib.x2g_relax_batch(self.ctx.h, self.gh, self.arr, self.n, maxsor1, maxsor2))
+        return self.ctx.counts()[STAGED] - before, self.f.get().reshape(self.n, -1)
+
+
+# one workgroup per grid, fronts, level tables (their one ordering), the
+# strip sweep of either precision
+@pytest.mark.parametrize("kw", [
+    dict(nni=61, nmu=91, count=4), dict(nni=61, nmu=91, count=4, method=1, ordering=1),
+    dict(nni=61, nmu=91, count=4, method=1, ordering=2), dict(nni=169, nmu=241, count=2),
+    dict(nni=61, nmu=91, count=4, prec=1),
+])
+def test_macro_iterations_stage_nothing(kw):
+    from x2dhf_amd import gpu
+    print(kw, flush=True)
+    with gpu.Context(0) as ctx:
+        b = Batch(ctx, **kw)
+        b.relax(1, 2)  # tunes the plan, builds the tables
+        one, _ = b.relax(1, 2)
+        many, got = b.relax(7, 2)
+        assert many == one, (one, many)
+        # seven macro-iterations in one call: as seven calls
+        b.f.set(b.u)
+        for _ in range(7):
+            gpu.check(ctx.lib.x2g_relax_batch(ctx.h, b.gh, b.arr, b.n, 1, 2))
+        assert np.array_equal(b.f.get().reshape(b.n, -1), got)
+        b.grid.destroy()

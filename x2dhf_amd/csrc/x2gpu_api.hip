@@ -75,6 +75,7 @@ int pinned_out_reserve(x2g_ctx *ctx, size_t bytes)
 
 int stage_bytes(x2g_ctx *ctx, const void *src, size_t bytes, const void **dev_out)
 {
+    ctx->counts[X2G_COUNT_STAGED] += (long long)bytes;
     if (ctx->cap_arena) {
         // graph capture: the descriptors belong to the graph's own arena
         const size_t off = (ctx->cap_off + 255) & ~size_t(255);

@@ -17,8 +17,18 @@ struct FrontItem {
 bool front_fits(const x2g_ctx *ctx, int nni, int nmu, int method, int ordering);
 // Reserve the workspace of launch_fronts.
 int front_reserve(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps);
-// nsweeps sweeps of every item (each must fit, and the workspace be reserved).
-int launch_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps);
+// Launches of nsweeps sweeps of every item (each must fit, and the workspace
+// be reserved), their descriptors staged.
+struct FrontDesc;
+struct FrontPlan {
+    const FrontDesc *descs = nullptr;
+    int n = 0, nsweeps = 0, threads = 0, most = 0;   // most: elements of the longest array by level
+    size_t lds = 0;
+    double bytes = 0;          // algorithmic, of one sweep
+};
+int plan_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps, FrontPlan &plan);
+// The sweeps.  Stages nothing, so it can run any number of times in a call.
+int launch_fronts(x2g_ctx *ctx, const FrontPlan &plan);
 int front_lds_attr(x2g_ctx *ctx);
 
 }  // namespace x2g

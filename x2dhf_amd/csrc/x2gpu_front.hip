@@ -441,15 +441,12 @@ int front_reserve(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps
     return ws_reserve(ctx, 4, off);
 }
 
-int launch_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps)
+int plan_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps, FrontPlan &plan)
 {
+    plan = FrontPlan{};
     if (items.empty() || nsweeps <= 0) return X2G_OK;
-    int rc;
     std::vector<FrontDesc> v;
     size_t off = 256;
-    int nt = 0, most = 0;
-    size_t lds = 0;
-    double bytes = 0;
     char *base = (char *)ctx->ws[4].ptr;
     for (auto &it : items) {
         const x2g_grid *g = it.g;
@@ -470,27 +467,36 @@ int launch_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps
         d.ls = d.rs + n;
         d.done = (unsigned *)(base + off + align256(3 * n * sizeof(double)));
         off += front_bytes(d, nsweeps);
-        nt = std::max(nt, front_threads(d.nni, d.nst));
-        lds = std::max(lds, front_lds(d));
-        most = std::max(most, (int)n);
-        bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5) * nsweeps;
+        plan.threads = std::max(plan.threads, front_threads(d.nni, d.nst));
+        plan.lds = std::max(plan.lds, front_lds(d));
+        plan.most = std::max(plan.most, (int)n);
+        plan.bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5);
         v.push_back(d);
     }
-    X2G_CHECK(ctx->ws[4].bytes >= off, "launch_fronts: workspace");
-    unsigned *tickets = (unsigned *)base;
-    const FrontDesc *dd;
-    if ((rc = stage_n(ctx, v.data(), v.size(), &dd)) || (rc = stage_flush(ctx))) return rc;
+    X2G_CHECK(ctx->ws[4].bytes >= off, "plan_fronts: workspace");
+    plan.n = (int)v.size();
+    plan.nsweeps = nsweeps;
+    return stage_n(ctx, v.data(), v.size(), &plan.descs);
+}
+
+int launch_fronts(x2g_ctx *ctx, const FrontPlan &plan)
+{
+    if (plan.n == 0) return X2G_OK;
+    int rc = stage_flush(ctx);
+    if (rc) return rc;
     hipEvent_t ea, eb;
     if ((rc = stats_begin(ctx, &ea, &eb))) return rc;
-    const int np = (int)v.size(), bx = std::min((most + 255) / 256, 1024);
-    X2G_LAUNCH(ctx, k_front_in, dim3(bx, np), dim3(256), 0, dd, tickets, nsweeps);
-    const dim3 wgs((unsigned)np * (unsigned)nsweeps);
-    if (nt <= 512) X2G_LAUNCH(ctx, k_front<512>, wgs, dim3(nt), lds, dd, tickets, np);
-    else if (nt <= 768) X2G_LAUNCH(ctx, k_front<768>, wgs, dim3(nt), lds, dd, tickets, np);
-    else X2G_LAUNCH(ctx, k_front<1024>, wgs, dim3(nt), lds, dd, tickets, np);
+    const FrontDesc *dd = plan.descs;
+    unsigned *tickets = (unsigned *)ctx->ws[4].ptr;
+    const int np = plan.n, nt = plan.threads, bx = std::min((plan.most + 255) / 256, 1024);
+    X2G_LAUNCH(ctx, k_front_in, dim3(bx, np), dim3(256), 0, dd, tickets, plan.nsweeps);
+    const dim3 wgs((unsigned)np * (unsigned)plan.nsweeps);
+    if (nt <= 512) X2G_LAUNCH(ctx, k_front<512>, wgs, dim3(nt), plan.lds, dd, tickets, np);
+    else if (nt <= 768) X2G_LAUNCH(ctx, k_front<768>, wgs, dim3(nt), plan.lds, dd, tickets, np);
+    else X2G_LAUNCH(ctx, k_front<1024>, wgs, dim3(nt), plan.lds, dd, tickets, np);
     X2G_LAUNCH(ctx, k_front_out, dim3(bx, np), dim3(256), 0, dd);
     X2G_HIP(hipGetLastError());
-    return stats_end(ctx, ea, eb, bytes, 0, nsweeps);
+    return stats_end(ctx, ea, eb, plan.bytes * plan.nsweeps, 0, plan.nsweeps);
 }
 
 }  // namespace x2g

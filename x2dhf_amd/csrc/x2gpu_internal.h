@@ -63,6 +63,7 @@ struct x2g_ctx {
     struct Pending { hipEvent_t a, b; double bytes; int prec, launches; };
     std::vector<Pending> pending;
     double st_launch[2] = {0, 0}, st_ms[2] = {0, 0}, st_bytes[2] = {0, 0};
+    long long counts[X2G_COUNTS] = {};  // x2g_call_counts
     // device blocks of x2g_malloc: sizes of the live ones, and freed ones
     // kept for reuse by size (all work on them is ordered by `stream`)
     std::unordered_map<void *, size_t> live;

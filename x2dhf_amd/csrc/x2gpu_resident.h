@@ -15,8 +15,17 @@ struct ResidentDesc {
 bool resident_fits(const x2g_ctx *ctx, int nni, int nmu);
 // Everything of a problem but its arrays.
 ResidentDesc resident_desc(const x2g_grid *g, int bkind, int isym, double omega);
-// nsweeps sweeps of every problem (each must fit).
-int launch_resident(x2g_ctx *ctx, std::vector<ResidentDesc> &v, int nsweeps);
+// A launch of all problems (each must fit), its descriptors staged.
+struct ResidentPlan {
+    const ResidentDesc *descs = nullptr;
+    int n = 0, groups = 1, threads = 64;
+    size_t lds = 0;
+    double bytes = 0;          // algorithmic, of one sweep
+};
+int plan_resident(x2g_ctx *ctx, std::vector<ResidentDesc> &v, ResidentPlan &plan);
+// nsweeps sweeps of every problem.  Stages nothing, so it can run any number
+// of times in a call.
+int launch_resident(x2g_ctx *ctx, const ResidentPlan &plan, int nsweeps);
 int resident_lds_attr(x2g_ctx *ctx);
 
 }  // namespace x2g

@@ -165,33 +165,38 @@ int resident_lds_attr(x2g_ctx *ctx)
     return X2G_OK;
 }
 
-int launch_resident(x2g_ctx *ctx, std::vector<ResidentDesc> &v, int nsweeps)
+int plan_resident(x2g_ctx *ctx, std::vector<ResidentDesc> &v, ResidentPlan &plan)
 {
-    if (v.empty() || nsweeps <= 0) return X2G_OK;
-    int G = 1, nt = 64;
-    size_t lds = 0;
-    double bytes = 0;
-    for (auto &d : v) G = std::max(G, res_pick(d.nni, d.nmu));
+    plan = ResidentPlan{};
+    if (v.empty()) return X2G_OK;
+    for (auto &d : v) plan.groups = std::max(plan.groups, res_pick(d.nni, d.nmu));
     for (auto &d : v) {
-        d.per = res_per(d.nni, G);
-        nt = std::max(nt, ((d.nmu - 5) * d.per + 63) & ~63);
-        lds = std::max(lds, res_lds(d.nni, d.nmu));
-        bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5) * nsweeps;
+        d.per = res_per(d.nni, plan.groups);
+        plan.threads = std::max(plan.threads, ((d.nmu - 5) * d.per + 63) & ~63);
+        plan.lds = std::max(plan.lds, res_lds(d.nni, d.nmu));
+        plan.bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5);
     }
-    const ResidentDesc *dd;
-    int rc;
-    if ((rc = stage_n(ctx, v.data(), v.size(), &dd)) || (rc = stage_flush(ctx))) return rc;
+    plan.n = (int)v.size();
+    return stage_n(ctx, v.data(), v.size(), &plan.descs);
+}
+
+int launch_resident(x2g_ctx *ctx, const ResidentPlan &plan, int nsweeps)
+{
+    if (plan.n == 0 || nsweeps <= 0) return X2G_OK;
+    int rc = stage_flush(ctx);
+    if (rc) return rc;
     hipEvent_t ea, eb;
     if ((rc = stats_begin(ctx, &ea, &eb))) return rc;
-    const dim3 wgs((unsigned)v.size()), th((unsigned)nt);
-    switch (G) {
-    case 1: X2G_LAUNCH(ctx, k_resident<1>, wgs, th, lds, dd, nsweeps); break;
-    case 2: X2G_LAUNCH(ctx, k_resident<2>, wgs, th, lds, dd, nsweeps); break;
-    case 3: X2G_LAUNCH(ctx, k_resident<3>, wgs, th, lds, dd, nsweeps); break;
-    default: X2G_LAUNCH(ctx, k_resident<4>, wgs, th, lds, dd, nsweeps); break;
+    const dim3 wgs((unsigned)plan.n), th((unsigned)plan.threads);
+    const ResidentDesc *dd = plan.descs;
+    switch (plan.groups) {
+    case 1: X2G_LAUNCH(ctx, k_resident<1>, wgs, th, plan.lds, dd, nsweeps); break;
+    case 2: X2G_LAUNCH(ctx, k_resident<2>, wgs, th, plan.lds, dd, nsweeps); break;
+    case 3: X2G_LAUNCH(ctx, k_resident<3>, wgs, th, plan.lds, dd, nsweeps); break;
+    default: X2G_LAUNCH(ctx, k_resident<4>, wgs, th, plan.lds, dd, nsweeps); break;
     }
     X2G_HIP(hipGetLastError());
-    return stats_end(ctx, ea, eb, bytes, 0, nsweeps);
+    return stats_end(ctx, ea, eb, plan.bytes * nsweeps, 0, nsweeps);
 }
 
 }  // namespace x2g

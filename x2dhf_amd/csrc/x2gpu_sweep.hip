@@ -2703,14 +2703,13 @@ static void fill_level_desc(LevelDesc &d, x2g_grid *g, const x2g_levels *L, doub
     d.lag = L->lag;
 }
 
-// nsweeps ordered sweeps of every problem in v (one workgroup each).
-static int launch_levels(x2g_ctx *ctx, const std::vector<LevelDesc> &v, int nsweeps)
+// nsweeps ordered sweeps of every problem in v (one workgroup each), whose
+// descriptors are staged at dd.
+static int launch_levels(x2g_ctx *ctx, const LevelDesc *dd, const std::vector<LevelDesc> &v, int nsweeps)
 {
     if (v.empty() || nsweeps <= 0) return X2G_OK;
-    const LevelDesc *dd;
-    int rc = stage_n(ctx, v.data(), v.size(), &dd);
+    int rc = stage_flush(ctx);
     if (rc) return rc;
-    if ((rc = stage_flush(ctx))) return rc;
     double bytes = 0.0;
     for (auto &d : v) bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5) * nsweeps;
     hipEvent_t ea, eb;
@@ -2875,7 +2874,9 @@ static int mcsor_run(x2g_grid *g, int isym, int bkind, double *work_d, const dou
         std::vector<ResidentDesc> v{resident_desc(g, bkind, isym, omega)};
         v[0].work = work_d;
         v[0].lr = lr;
-        return launch_resident(ctx, v, nsweeps);
+        ResidentPlan plan;
+        if ((rc = plan_resident(ctx, v, plan))) return rc;
+        return launch_resident(ctx, plan, nsweeps);
     }
     const bool restride = kind == 2;
     double *A = work_d, *B = (double *)w0;
@@ -2972,15 +2973,18 @@ extern "C" int x2g_relax_ordered(x2g_grid *g, int isym, int bkind, double *work_
     if (levels_pipe() && front_fits(g->ctx, g->nni, g->nmu, method, ordering)) {
         const std::vector<FrontItem> fv = {{g, work_d, lhs_d, rhs_d, omega, bkind, isym, method, ordering}};
         if (front_reserve(g->ctx, fv, nsweeps) == X2G_OK) {
-            if ((rc = set_lds_attr(g->ctx))) return rc;
-            return launch_fronts(g->ctx, fv, nsweeps);
+            FrontPlan plan;
+            if ((rc = set_lds_attr(g->ctx)) || (rc = plan_fronts(g->ctx, fv, nsweeps, plan))) return rc;
+            return launch_fronts(g->ctx, plan);
         }
     }
     const x2g_levels *L;
     if ((rc = grid_levels(g, method, ordering, &L))) return rc;
     std::vector<LevelDesc> v(1);
     fill_level_desc(v[0], g, L, work_d, lhs_d, rhs_d, bkind, isym, omega);
-    return launch_levels(g->ctx, v, nsweeps);
+    const LevelDesc *dd;
+    if ((rc = stage_n(g->ctx, v.data(), v.size(), &dd))) return rc;
+    return launch_levels(g->ctx, dd, v, nsweeps);
 }
 
 extern "C" int x2g_mcsor_host(x2g_grid *g, int isym, int bkind, double *work, const double *lhs,
@@ -3181,7 +3185,7 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
     // FP64 items: sweep plan
     SweepPlan<double> p64;
     const SweepDesc<double> *d64e = nullptr, *d64o = nullptr;
-    std::vector<ResidentDesc> res64;
+    ResidentPlan res64;
     std::vector<PadDesc> pout64;
     if (!i64.empty()) {
         std::vector<SweepDesc<double>> base(i64.size());
@@ -3208,12 +3212,14 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
             if ((rc = launch_pack(ctx, pk))) return rc;
         }
         if (kind64 == 4) {
+            std::vector<ResidentDesc> rv;
             for (size_t k = 0; k < i64.size(); ++k) {
                 const x2g_relax_item &it = items[i64[k]];
-                res64.push_back(resident_desc(grids[it.grid_index], it.bkind, it.isym, it.omega));
-                res64.back().work = A[k];
-                res64.back().lr = lrp(i64[k]);
+                rv.push_back(resident_desc(grids[it.grid_index], it.bkind, it.isym, it.omega));
+                rv.back().work = A[k];
+                rv.back().lr = lrp(i64[k]);
             }
+            if ((rc = plan_resident(ctx, rv, res64))) return rc;
         } else {
             SweepKnobs kn64;
             if ((rc = tuned_knobs<double>(ctx, base, A, B, false, kn64))) return rc;
@@ -3260,6 +3266,12 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
         }
         pout_ord.push_back({it.fun_d, bufA(i), nullptr, g->nni, g->nmu, 1, g->nni + 8});
     }
+    // the macro-iterations below stage nothing: what a call stages does not
+    // grow with their number
+    const LevelDesc *d_lev = nullptr;
+    FrontPlan pfront;
+    if (!lev.empty() && (rc = stage_descs(ctx, lev, doff, &d_lev))) return rc;
+    if ((rc = plan_fronts(ctx, fronts, maxsor2, pfront))) return rc;
     const PadDesc *d_pout_ord = nullptr;
     if (!pout_ord.empty() && (rc = stage_descs(ctx, pout_ord, doff, &d_pout_ord))) return rc;
 
@@ -3403,8 +3415,8 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
             X2G_HIP(hipGetLastError());
         }
         if (!iord.empty() && maxsor2 > 0) {
-            if ((rc = launch_levels(ctx, lev, maxsor2))) return rc;
-            if ((rc = launch_fronts(ctx, fronts, maxsor2))) return rc;
+            if ((rc = launch_levels(ctx, d_lev, lev, maxsor2))) return rc;
+            if ((rc = launch_fronts(ctx, pfront))) return rc;
             X2G_LAUNCH(ctx, k_putout, dim3(grid_x_for(maxn, 256), (int)iord.size()), dim3(256), 0,
                                d_pout_ord);
             X2G_HIP(hipGetLastError());
@@ -3607,6 +3619,13 @@ extern "C" int x2g_graph_counts(x2g_ctx *ctx, long long *captures, long long *re
     X2G_CHECK(ctx && captures && replays, "x2g_graph_counts: null argument");
     *captures = ctx->graph_captures;
     *replays = ctx->graph_replays;
+    return X2G_OK;
+}
+
+extern "C" int x2g_call_counts(x2g_ctx *ctx, long long *out, int n)
+{
+    X2G_CHECK(ctx && out && n >= 0, "x2g_call_counts: null argument");
+    for (int k = 0; k < n; ++k) out[k] = k < X2G_COUNTS ? ctx->counts[k] : 0;
     return X2G_OK;
 }
 

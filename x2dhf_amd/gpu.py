@@ -106,6 +106,7 @@ _PROTOS = {
     "x2g_mem_info": (_int, [_vp, C.POINTER(_szt), C.POINTER(_szt)]),
     "x2g_stats_enable": (_int, [_vp, _int]),
     "x2g_stats_get": (_int, [_vp, _vp]),
+    "x2g_call_counts": (_int, [_vp, C.POINTER(C.c_longlong), _int]),
     "x2g_malloc": (_int, [_vp, _szt, C.POINTER(_vp)]),
     "x2g_free": (_int, [_vp, _vp]),
     "x2g_h2d": (_int, [_vp, _vp, _vp, _szt]),
@@ -215,6 +216,12 @@ class Context:
 
     def __exit__(self, *a):
         self.close()
+
+    def counts(self, n=16):
+        """x2g_call_counts: what the calls on this context did so far."""
+        out = (C.c_longlong * n)()
+        check(self.lib.x2g_call_counts(self.h, out, n))
+        return list(out)
 
     def sync(self):
         check(self.lib.x2g_ctx_sync(self.h))

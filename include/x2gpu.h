@@ -84,9 +84,20 @@ int x2g_stats_enable(x2g_ctx *ctx, int on);
 int x2g_stats_get(x2g_ctx *ctx, double *out);
 
 /* What the calls on this context did so far, out[X2G_COUNT_*] for the first n
- * counts (those past the last are 0): bytes of launch descriptors staged. */
+ * counts (those past the last are 0): bytes of launch descriptors staged, and
+ * launches of each relaxation kernel.  A captured call counts as it is
+ * recorded, a replay of its graph counts nothing; the autotuner's trial
+ * launches count too. */
 #define X2G_COUNT_STAGED 0
-#define X2G_COUNTS 1
+#define X2G_COUNT_PHASE 1      /* a launch per colour pass */
+#define X2G_COUNT_STRIP 2      /* the first pipelined strip kernel */
+#define X2G_COUNT_SWEEP64 3    /* the strip sweep, FP64 */
+#define X2G_COUNT_SWEEP32 4    /* the strip sweep, FP32 */
+#define X2G_COUNT_CHAIN 5      /* several FP32 sweeps of a large batch */
+#define X2G_COUNT_RESIDENT 6   /* all FP64 sweeps of small grids */
+#define X2G_COUNT_FRONT 7      /* all ordered SOR sweeps, a workgroup per sweep */
+#define X2G_COUNT_LEVELS 8     /* all ordered sweeps, a workgroup per problem */
+#define X2G_COUNTS 9
 int x2g_call_counts(x2g_ctx *ctx, long long *out, int n);
 
 /* ---- device memory ------------------------------------------------------ */

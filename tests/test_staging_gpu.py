@@ -10,8 +10,6 @@ from test_kernels_gpu import synthetic_problem
 
 pytestmark = pytest.mark.gpu
 
-STAGED = 0  # X2G_COUNT_STAGED
-
 
 class Batch:
     """count functions of one grid as relax items of one scheme."""
@@ -36,9 +34,9 @@ class Batch:
         """Bytes staged by one call from the starting functions; the results."""
         from x2dhf_amd import gpu
         self.f.set(self.u)
-        before = self.ctx.counts()[STAGED]
+        before = self.ctx.counts()["staged"]
         gpu.check(self.ctx.lib.x2g_relax_batch(self.ctx.h, self.gh, self.arr, self.n, maxsor1, maxsor2))
-        return self.ctx.counts()[STAGED] - before, self.f.get().reshape(self.n, -1)
+        return self.ctx.counts()["staged"] - before, self.f.get().reshape(self.n, -1)
 
 
 # one workgroup per grid, fronts, level tables (their one ordering), the

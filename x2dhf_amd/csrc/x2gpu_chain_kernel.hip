@@ -54,6 +54,7 @@ int chain_kernel(x2g_ctx *ctx, const ChainPack *packs, const ChainSeg *segs, con
                  int sweeps, int first)
 {
     X2G_LAUNCH(ctx, k_chain_f32, dim3(nwg), dim3(64 * kChainWaves), 0, packs, segs, wgs, sweeps, first);
+    ++ctx->counts[X2G_COUNT_CHAIN];
     X2G_HIP(hipGetLastError());
     return X2G_OK;
 }

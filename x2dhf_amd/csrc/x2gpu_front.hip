@@ -494,6 +494,7 @@ int launch_fronts(x2g_ctx *ctx, const FrontPlan &plan)
     if (nt <= 512) X2G_LAUNCH(ctx, k_front<512>, wgs, dim3(nt), plan.lds, dd, tickets, np);
     else if (nt <= 768) X2G_LAUNCH(ctx, k_front<768>, wgs, dim3(nt), plan.lds, dd, tickets, np);
     else X2G_LAUNCH(ctx, k_front<1024>, wgs, dim3(nt), plan.lds, dd, tickets, np);
+    ++ctx->counts[X2G_COUNT_FRONT];
     X2G_LAUNCH(ctx, k_front_out, dim3(bx, np), dim3(256), 0, dd);
     X2G_HIP(hipGetLastError());
     return stats_end(ctx, ea, eb, plan.bytes * plan.nsweeps, 0, plan.nsweeps);

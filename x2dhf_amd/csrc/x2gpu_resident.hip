@@ -195,6 +195,7 @@ int launch_resident(x2g_ctx *ctx, const ResidentPlan &plan, int nsweeps)
     case 3: X2G_LAUNCH(ctx, k_resident<3>, wgs, th, plan.lds, dd, nsweeps); break;
     default: X2G_LAUNCH(ctx, k_resident<4>, wgs, th, plan.lds, dd, nsweeps); break;
     }
+    ++ctx->counts[X2G_COUNT_RESIDENT];
     X2G_HIP(hipGetLastError());
     return stats_end(ctx, ea, eb, plan.bytes * nsweeps, 0, nsweeps);
 }

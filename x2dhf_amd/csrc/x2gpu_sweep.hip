@@ -1891,6 +1891,7 @@ static int launch_sweep_once(x2g_ctx *ctx, const SweepDesc<T> *dd, const std::ve
         for (const auto &sub : plan.subs) {
             const bool ok = dispatch_ks<T>(ctx, dd, sub, zero_src ? 1 : 0);
             X2G_CHECK(ok, "no sweep kernel for ring stride %d", sub.W);
+            ++ctx->counts[sizeof(T) == 8 ? X2G_COUNT_SWEEP64 : X2G_COUNT_SWEEP32];
             X2G_HIP(hipGetLastError());
         }
         return X2G_OK;
@@ -1902,6 +1903,7 @@ static int launch_sweep_once(x2g_ctx *ctx, const SweepDesc<T> *dd, const std::ve
         } else {
             X2G_LAUNCH(ctx, (k_strip<T, 1>), dim3(total_wg), dim3(nth), lds, dd, n);
         }
+        ++ctx->counts[X2G_COUNT_STRIP];
         X2G_HIP(hipGetLastError());
         return X2G_OK;
     }
@@ -1909,6 +1911,7 @@ static int launch_sweep_once(x2g_ctx *ctx, const SweepDesc<T> *dd, const std::ve
     for (auto &d : hv) maxpts = std::max<long>(maxpts, (long)(d.nni - 2) * (d.nmu - 5));
     for (int pass = 0; pass < 5; ++pass) {
         X2G_LAUNCH(ctx, (k_phase<T>), dim3(grid_x_for(maxpts, 256), n), dim3(256), 0, dd, pass);
+        ++ctx->counts[X2G_COUNT_PHASE];
         X2G_HIP(hipGetLastError());
     }
     long maxb = 0;
@@ -2718,6 +2721,7 @@ static int launch_levels(x2g_ctx *ctx, const LevelDesc *dd, const std::vector<Le
         X2G_LAUNCH(ctx, k_levels_pipe, dim3((int)v.size()), dim3(kPipeThreads), 0, dd, nsweeps);
     else
         X2G_LAUNCH(ctx, k_levels, dim3((int)v.size()), dim3(kLevelThreads), 0, dd, nsweeps);
+    ++ctx->counts[X2G_COUNT_LEVELS];
     X2G_HIP(hipGetLastError());
     return stats_end(ctx, ea, eb, bytes, 0, nsweeps);
 }

@@ -95,6 +95,9 @@ class ScfCtrl(C.Structure):
                 ("mm_due", _int), ("prec", _int), ("polish_end", _int), ("stopcode", _int), ("stop", _int)]
 
 
+# X2G_COUNT_*: bytes of descriptors staged, then launches by kernel
+COUNTS = ("staged", "phase", "strip", "sweep64", "sweep32", "chain", "resident", "front", "levels")
+
 # name -> (restype, argtypes)
 _PROTOS = {
     "x2g_version": (_int, []),
@@ -217,11 +220,11 @@ class Context:
     def __exit__(self, *a):
         self.close()
 
-    def counts(self, n=16):
-        """x2g_call_counts: what the calls on this context did so far."""
-        out = (C.c_longlong * n)()
-        check(self.lib.x2g_call_counts(self.h, out, n))
-        return list(out)
+    def counts(self):
+        """x2g_call_counts: what the calls on this context did so far, by name."""
+        out = (C.c_longlong * len(COUNTS))()
+        check(self.lib.x2g_call_counts(self.h, out, len(COUNTS)))
+        return dict(zip(COUNTS, out))
 
     def sync(self):
         check(self.lib.x2g_ctx_sync(self.h))

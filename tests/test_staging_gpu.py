@@ -61,3 +61,26 @@ def test_macro_iterations_stage_nothing(kw):
             gpu.check(ctx.lib.x2g_relax_batch(ctx.h, b.gh, b.arr, b.n, 1, 2))
         assert np.array_equal(b.f.get().reshape(b.n, -1), got)
         b.grid.destroy()
+
+
+def test_more_chained_sweeps_stage_nothing_more():
+    """400 sweeps of a large FP32 batch stage what 200 do, and leave what one
+    launch per sweep leaves (an odd number, so that a launch is shorter)."""
+    from x2dhf_amd import gpu
+    with gpu.Context(0) as ctx:
+        b = Batch(ctx, 91, 121, 350, prec=1)
+        out = {}
+        for sweeps in (200, 400, 401):
+            print(sweeps, flush=True)
+            n = ctx.counts()["chain"]
+            out[sweeps] = b.relax(1, sweeps)
+            n = ctx.counts()["chain"] - n
+            assert n > 1 and n < sweeps
+        assert out[400][0] == out[200][0], (out[200][0], out[400][0])
+        gpu.check(ctx.lib.x2g_set_sweep_plan(4, 0, 0))
+        try:
+            _, want = b.relax(1, 401)
+        finally:
+            gpu.check(ctx.lib.x2g_set_sweep_plan(0, 0, 0))
+        assert np.array_equal(out[401][1], want)
+        b.grid.destroy()

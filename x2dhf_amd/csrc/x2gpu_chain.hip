@@ -2,6 +2,8 @@
 // workgroups and launches of a batch.
 #include "x2gpu_chain.h"
 #include <algorithm>
+#include <map>
+#include <tuple>
 
 namespace x2g {
 
@@ -166,10 +168,18 @@ int chain_plan(x2g_ctx *ctx, const std::vector<ChainProblem> &probs, int nsweeps
     const int nch = (nsweeps + cut.sweeps - 1) / cut.sweeps;
     plan.out.resize(probs.size());
     int done = 0;
+    // Launches of one direction and length have the same descriptors, which are
+    // staged once: what a plan stages does not grow with its sweeps.
+    std::map<std::tuple<bool, bool, int, int>, ChainPlan::Chunk> staged;
     for (int k = 0; k < nch; ++k) {
         ChainPlan::Chunk ck{};
         ck.sweeps = (nsweeps - done + nch - k - 1) / (nch - k);
         done += ck.sweeps;
+        const auto key = std::make_tuple(k == 0, k == nch - 1, k % 2, ck.sweeps);
+        if (const auto it = staged.find(key); it != staged.end()) {
+            plan.chunks.push_back(it->second);
+            continue;
+        }
         std::vector<ChainPack> packs;
         std::vector<ChainSeg> segs;
         std::vector<ChainWg> wgs;
@@ -229,6 +239,7 @@ int chain_plan(x2g_ctx *ctx, const std::vector<ChainProblem> &probs, int nsweeps
         if ((rc = stage_n(ctx, segs.data(), segs.size(), &ck.segs))) return rc;
         if ((rc = stage_n(ctx, wgs.data(), wgs.size(), &ck.wgs))) return rc;
         plan.chunks.push_back(ck);
+        staged[key] = ck;
     }
     return X2G_OK;
 }

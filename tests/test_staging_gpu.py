@@ -38,6 +38,13 @@ class Batch:
         gpu.check(self.ctx.lib.x2g_relax_batch(self.ctx.h, self.gh, self.arr, self.n, maxsor1, maxsor2))
         return self.ctx.counts()["staged"] - before, self.f.get().reshape(self.n, -1)
 
+    def relax_first(self, count):
+        """As relax(2, 2) of the first `count` functions."""
+        from x2dhf_amd import gpu
+        self.f.set(self.u)
+        gpu.check(self.ctx.lib.x2g_relax_batch(self.ctx.h, self.gh, self.arr, count, 2, 2))
+        return self.f.get().reshape(len(self.u), -1)
+
 
 # one workgroup per grid, fronts, level tables (their one ordering), the
 # strip sweep of either precision
@@ -83,4 +90,31 @@ def test_more_chained_sweeps_stage_nothing_more():
         finally:
             gpu.check(ctx.lib.x2g_set_sweep_plan(0, 0, 0))
         assert np.array_equal(out[401][1], want)
+        b.grid.destroy()
+
+
+def test_descriptors_of_one_call_beyond_the_ring():
+    """45 000 ordered functions in one call: their descriptors take more than
+    the 16 MiB ring, and the first staged are read again in the second
+    macro-iteration.  Then a small call, which gives the outgrown ring back."""
+    from x2dhf_amd import gpu
+    nni, nmu, n = 24, 24, 45000
+    with gpu.Context(0) as ctx:
+        b = Batch(ctx, nni, nmu, n, method=1, ordering=0)
+        P, want = b.P, []
+        for k in range(5):
+            u = b.u[k]
+            for _ in range(2):
+                w = pyoracle.putin(nni, nmu, 1, u)
+                pyoracle.relax_ordered(nni, nmu, 1, w, P["lhs"], P["rhs"], P["suppl"][1], P["suppl"][2],
+                                       P["coef"][:16], P["coef"][16:21], 1.8, 2, 1, "col-wise")
+                u = pyoracle.putout(nni, nmu, w)
+            want.append(u)
+        print(f"{n} items", flush=True)
+        staged, got = b.relax(2, 2)
+        assert staged > 16 << 20
+        assert np.array_equal(got.reshape(n // 5, 5, -1), np.broadcast_to(want, (n // 5, 5, nni * nmu)))
+        for count in (7, n, 7):
+            got = b.relax_first(count)
+            assert np.array_equal(got[:count], np.tile(want, (n // 5, 1))[:count]), count
         b.grid.destroy()

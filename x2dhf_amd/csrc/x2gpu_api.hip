@@ -73,6 +73,63 @@ int pinned_out_reserve(x2g_ctx *ctx, size_t bytes)
     return X2G_OK;
 }
 
+static constexpr size_t kStageBytes = 16u << 20;  // launch-descriptor staging ring
+
+// Every copy and launch that used the ring has to be done: start it over.
+static int stage_wrap(x2g_ctx *ctx)
+{
+    const int rc = stage_flush(ctx);
+    if (rc) return rc;
+    X2G_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->stage_off = 0;
+    return X2G_OK;
+}
+
+void stage_free_old(x2g_ctx *ctx)
+{
+    for (auto &o : ctx->stage_old) {
+        (void)hipFree(o.first);
+        (void)hipHostFree(o.second);
+    }
+    ctx->stage_old.clear();
+}
+
+// Replace the ring, which the running call still reads, by one of twice its size.
+static int stage_grow(x2g_ctx *ctx)
+{
+    const int rc = stage_flush(ctx);
+    if (rc) return rc;
+    const size_t want = 2 * std::min(ctx->ws[2].bytes, ctx->pinned_bytes);
+    void *dev = nullptr, *host = nullptr;
+    if (hipMalloc(&dev, want) != hipSuccess || hipHostMalloc(&host, want, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        if (dev) (void)hipFree(dev);
+        set_error("launch descriptors: a ring of %zu bytes could not be allocated", want);
+        return X2G_ENOMEM;
+    }
+    ctx->stage_old.push_back({ctx->ws[2].ptr, ctx->pinned});
+    ctx->ws[2].ptr = dev;
+    ctx->pinned = host;
+    ctx->ws[2].bytes = ctx->pinned_bytes = want;
+    ctx->stage_off = 0;
+    return X2G_OK;
+}
+
+int stage_call_begin(x2g_ctx *ctx)
+{
+    ctx->stage_used = 0;
+    if (ctx->cap_arena) return X2G_OK;   // a capture has its arena
+    // room for as much as any call took so far, or start over
+    const size_t cap = std::min(ctx->ws[2].bytes, ctx->pinned_bytes);
+    if (!ctx->stage_old.empty() || (ctx->stage_off && ctx->stage_off + ctx->stage_peak > cap)) {
+        const int rc = stage_wrap(ctx);
+        if (rc) return rc;
+        stage_free_old(ctx);
+    }
+    ctx->stage_call = true;
+    return X2G_OK;
+}
+
 int stage_bytes(x2g_ctx *ctx, const void *src, size_t bytes, const void **dev_out)
 {
     ctx->counts[X2G_COUNT_STAGED] += (long long)bytes;
@@ -89,15 +146,14 @@ int stage_bytes(x2g_ctx *ctx, const void *src, size_t bytes, const void **dev_ou
         return X2G_OK;
     }
     const size_t cap = std::min(ctx->ws[2].bytes, ctx->pinned_bytes);
-    X2G_CHECK(bytes <= cap, "launch descriptors (%zu bytes) exceed the staging ring", bytes);
+    X2G_CHECK(bytes <= kStageBytes, "launch descriptors (%zu bytes) exceed the staging ring", bytes);
     size_t off = (ctx->stage_off + 255) & ~size_t(255);
     if (off + bytes > cap) {
-        // wrap: every copy and launch that used the ring has to be done
-        const int rc = stage_flush(ctx);
+        const int rc = ctx->stage_call ? stage_grow(ctx) : stage_wrap(ctx);
         if (rc) return rc;
-        X2G_HIP(hipStreamSynchronize(ctx->stream));
         off = 0;
     }
+    ctx->stage_used += (bytes + 255) & ~size_t(255);
     std::memcpy((char *)ctx->pinned + off, src, bytes);
     if (ctx->stage_hi == ctx->stage_lo) ctx->stage_lo = off;
     ctx->stage_hi = off + bytes;
@@ -196,8 +252,6 @@ extern "C" int x2g_stats_get(x2g_ctx *ctx, double *out)
     return X2G_OK;
 }
 
-static constexpr size_t kStageBytes = 16u << 20;  // launch-descriptor staging ring
-
 extern "C" int x2g_version(void) { return 100; }
 
 extern "C" const char *x2g_last_error(void) { return x2g::g_err; }
@@ -265,6 +319,7 @@ extern "C" int x2g_ctx_destroy(x2g_ctx *ctx)
     for (auto &w : ctx->ws)
         if (w.ptr) (void)hipFree(w.ptr);
     for (auto &c : ctx->cache) (void)hipFree(c.second);
+    stage_free_old(ctx);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
     if (ctx->pinned_out) (void)hipHostFree(ctx->pinned_out);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

@@ -55,6 +55,9 @@ struct x2g_ctx {
     size_t pinned_out_bytes = 0;
     size_t stage_off = 0;          // ring offset into ws[2] / pinned
     size_t stage_lo = 0, stage_hi = 0;  // staged bytes not yet copied to ws[2]: [lo, hi)
+    bool stage_call = false;       // inside a StageCall: the ring does not wrap
+    size_t stage_used = 0, stage_peak = 0;  // bytes staged by this StageCall, and by the largest
+    std::vector<std::pair<void *, void *>> stage_old;  // outgrown rings (device, pinned) a call may still read
     // sweep-kernel timing (x2g_stats_enable): an event pair around each run of
     // back-to-back sweep launches, resolved at x2g_stats_get or when the
     // pending list is long
@@ -138,6 +141,24 @@ int pinned_reserve(x2g_ctx *ctx, size_t bytes);
 // stage_flush).  A region is reused only after the stream has been
 // synchronised past its last use.
 int stage_bytes(x2g_ctx *ctx, const void *src, size_t bytes, const void **dev_out);
+// The scope of a call that stages several arrays and reads the first of them
+// after the last was staged: inside it the ring is not wrapped over what the
+// call has staged, but replaced by a larger one (the old one lives until a
+// later call's scope begins).
+int stage_call_begin(x2g_ctx *ctx);
+void stage_free_old(x2g_ctx *ctx);
+struct StageCall {
+    x2g_ctx *ctx;
+    const int rc;
+    explicit StageCall(x2g_ctx *c) : ctx(c), rc(stage_call_begin(c)) {}
+    ~StageCall()
+    {
+        ctx->stage_call = false;
+        if (ctx->stage_used > ctx->stage_peak) ctx->stage_peak = ctx->stage_used;
+    }
+    StageCall(const StageCall &) = delete;
+    StageCall &operator=(const StageCall &) = delete;
+};
 // Issue one stream-ordered copy of everything staged since the last flush.
 int stage_flush(x2g_ctx *ctx);
 // Release every captured graph of the context.

@@ -806,8 +806,9 @@ extern "C" int x2g_lincomb_batch(x2g_ctx *ctx, x2g_grid *const *grids, const x2g
     size_t off = 0;
     const LcOp *dops;
     const x2g_term *dt = nullptr;
-    int rc = stage(ctx, v.data(), v.size(), off, &dops);
-    if (rc) return rc;
+    const StageCall staging(ctx);
+    int rc = staging.rc;
+    if (rc || (rc = stage(ctx, v.data(), v.size(), off, &dops))) return rc;
     if (nterms_total && (rc = stage(ctx, terms, (size_t)nterms_total, off, &dt))) return rc;
     const int nchunk = (int)((maxn + 256 * kLcIlp - 1) / (256 * kLcIlp)), slice = (nchunk + 7) / 8;
     X2G_LAUNCH(ctx, k_lincomb_batch, dim3(8 * nops * slice), dim3(256), 0, dops, dt, nops, nchunk, slice);

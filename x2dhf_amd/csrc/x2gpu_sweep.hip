@@ -3026,8 +3026,9 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
     X2G_CHECK(ctx && grids && (items || n == 0) && n >= 0, "x2g_relax_batch: null argument");
     X2G_CHECK(maxsor1 >= 0 && maxsor2 >= 0, "x2g_relax_batch: negative sweep counts");
     if (n == 0 || maxsor1 == 0) return X2G_OK;
-    int rc = set_lds_attr(ctx);
-    if (rc) return rc;
+    const StageCall staging(ctx);
+    int rc = staging.rc;
+    if (rc || (rc = set_lds_attr(ctx))) return rc;
     // validate, pick the sweep kind of each precision's batch (it fixes the
     // row stride of the padded arrays), and size the workspace: per FP64
     // item two padded arrays and the (omega/lhs, rhs) pairs; per FP32 item

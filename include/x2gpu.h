@@ -97,7 +97,8 @@ int x2g_stats_get(x2g_ctx *ctx, double *out);
 #define X2G_COUNT_RESIDENT 6   /* all FP64 sweeps of small grids */
 #define X2G_COUNT_FRONT 7      /* all ordered SOR sweeps, a workgroup per sweep */
 #define X2G_COUNT_LEVELS 8     /* all ordered sweeps, a workgroup per problem */
-#define X2G_COUNTS 9
+#define X2G_COUNT_WORKSPACE 9  /* bytes of relaxation workspace held now */
+#define X2G_COUNTS 10
 int x2g_call_counts(x2g_ctx *ctx, long long *out, int n);
 
 /* ---- device memory ------------------------------------------------------ */
@@ -301,12 +302,17 @@ int x2g_relax_batch(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_relax_item *
 
 /* Device workspace bytes (an upper bound) that one relaxation problem on an
  * nni x nmu grid of precision prec adds to the context's workspace while
- * x2g_relax_batch runs (padded sweep buffers and the colour-ordered
- * lhs/rhs pairs); the workspace is shared by the items of a call and kept
+ * x2g_relax_batch runs, in whichever scheme: padded sweep buffers and the
+ * colour-ordered lhs/rhs pairs, or, for the ordered SOR schemes that run a
+ * workgroup per sweep, a padded array and the function, lhs and rhs by
+ * dependency level.  The workspace is shared by the items of a call and kept
  * between calls.  No device call; -1 for bad sizes.  No reference
  * counterpart (the reference's per-thread temporaries,
  * c/relax_single_pot_pthread.c:65-67, are host mallocs). */
 long long x2g_relax_workspace_bytes(int nni, int nmu, int prec);
+/* The same for one scheme (method X2G_MCSOR .., ordering X2G_ORDER_*); -1 also
+ * for a bad scheme, and for prec = 1 with another than col-wise MCSOR. */
+long long x2g_relax_scheme_workspace_bytes(int nni, int nmu, int prec, int method, int ordering);
 
 /* FP64 residual norm^2 sum (rhs - A u)^2 over the relaxed interior of each
  * item, and sum rhs^2 (for relative residuals).  out[2*i], out[2*i+1]. */

@@ -25,7 +25,7 @@ class Ran:
 
     def __exit__(self, *a):
         self.n = {k: v - self.before[k] for k, v in self.ctx.counts().items()}
-        self.kernels = {k for k, v in self.n.items() if v and k != "staged"}
+        self.kernels = {k for k, v in self.n.items() if v and k not in ("staged", "workspace")}
 
 
 class Problems:

@@ -276,8 +276,7 @@ extern "C" int x2g_ctx_create(int device, x2g_ctx **out)
     int optin = 0;
     if (hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, device) != hipSuccess) optin = 0;
     size_t lds = std::max<size_t>((size_t)prop.sharedMemPerBlock, (size_t)std::max(optin, 0));
-    // gfx950 provides 160 KB of LDS per compute unit
-    c->max_lds = std::min<size_t>(lds, 160 * 1024);
+    c->max_lds = std::min<size_t>(lds, kMaxLds);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         delete c;
         set_error("hipStreamCreateWithFlags failed");

@@ -15,6 +15,9 @@ struct FrontItem {
 };
 // Whether (method, ordering) on a grid of nni x nmu runs as fronts.
 bool front_fits(const x2g_ctx *ctx, int nni, int nmu, int method, int ordering);
+// Bytes that one problem's fronts add to the workspace at most, however many
+// sweeps (0: does not run as fronts).
+size_t front_workspace_bytes(int nni, int nmu, int method, int ordering);
 // Reserve the workspace of launch_fronts.
 int front_reserve(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps);
 // Launches of nsweeps sweeps of every item (each must fit, and the workspace

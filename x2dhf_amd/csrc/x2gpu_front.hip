@@ -42,6 +42,7 @@ constexpr int kRowGap = 11;      // a row behind row 0 may be written this many 
 constexpr int kReach = 2 * kU + kAhead + kRowGap;   // levels that must be done before a block's loads
 constexpr int kFlagGap = 32;     // words between counters
 constexpr int kMinFront = 24;    // least nni, nmu
+constexpr int kFrontSweeps = 1024;   // sweeps of a launch at most: they bound the counters' memory
 
 enum { kStraight = 0, kReversed = 1, kMirrored = 2 };
 
@@ -407,13 +408,18 @@ static FrontDesc front_shape(int nni, int nmu, int method, int ordering)
     return d;
 }
 
-bool front_fits(const x2g_ctx *ctx, int nni, int nmu, int method, int ordering)
+static bool front_fits_lds(size_t max_lds, int nni, int nmu, int method, int ordering)
 {
     int rows, cols;
     if (!front_ways(method, ordering, rows, cols)) return false;
     const int nst = rows == kMirrored ? 2 : 1;
     return nni >= kMinFront && nmu >= kMinFront && (long)nmu * nni < (1L << 28) && front_threads(nni, nst) <= 1024 &&
-           front_lds(front_shape(nni, nmu, method, ordering)) + 64 <= ctx->max_lds;
+           front_lds(front_shape(nni, nmu, method, ordering)) + 64 <= max_lds;
+}
+
+bool front_fits(const x2g_ctx *ctx, int nni, int nmu, int method, int ordering)
+{
+    return front_fits_lds(ctx->max_lds, nni, nmu, method, ordering);
 }
 
 int front_lds_attr(x2g_ctx *ctx)
@@ -429,7 +435,14 @@ static size_t front_array(const FrontDesc &d) { return (size_t)d.nst * d.rows * 
 static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 static size_t front_bytes(const FrontDesc &d, int nsweeps)
 {
-    return align256(3 * front_array(d) * sizeof(double)) + align256((size_t)nsweeps * kFlagGap * sizeof(unsigned));
+    return align256(3 * front_array(d) * sizeof(double)) +
+           align256((size_t)std::min(nsweeps, kFrontSweeps) * kFlagGap * sizeof(unsigned));
+}
+
+size_t front_workspace_bytes(int nni, int nmu, int method, int ordering)
+{
+    if (!front_fits_lds(kMaxLds, nni, nmu, method, ordering)) return 0;
+    return 256 + front_bytes(front_shape(nni, nmu, method, ordering), kFrontSweeps);   // 256: the call's tickets
 }
 
 int front_reserve(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps)
@@ -489,14 +502,17 @@ int launch_fronts(x2g_ctx *ctx, const FrontPlan &plan)
     const FrontDesc *dd = plan.descs;
     unsigned *tickets = (unsigned *)ctx->ws[4].ptr;
     const int np = plan.n, nt = plan.threads, bx = std::min((plan.most + 255) / 256, 1024);
-    X2G_LAUNCH(ctx, k_front_in, dim3(bx, np), dim3(256), 0, dd, tickets, plan.nsweeps);
-    const dim3 wgs((unsigned)np * (unsigned)plan.nsweeps);
-    if (nt <= 512) X2G_LAUNCH(ctx, k_front<512>, wgs, dim3(nt), plan.lds, dd, tickets, np);
-    else if (nt <= 768) X2G_LAUNCH(ctx, k_front<768>, wgs, dim3(nt), plan.lds, dd, tickets, np);
-    else X2G_LAUNCH(ctx, k_front<1024>, wgs, dim3(nt), plan.lds, dd, tickets, np);
-    ++ctx->counts[X2G_COUNT_FRONT];
-    X2G_LAUNCH(ctx, k_front_out, dim3(bx, np), dim3(256), 0, dd);
-    X2G_HIP(hipGetLastError());
+    for (int done = 0; done < plan.nsweeps; done += kFrontSweeps) {
+        const int ns = std::min(plan.nsweeps - done, kFrontSweeps);
+        X2G_LAUNCH(ctx, k_front_in, dim3(bx, np), dim3(256), 0, dd, tickets, ns);
+        const dim3 wgs((unsigned)np * (unsigned)ns);
+        if (nt <= 512) X2G_LAUNCH(ctx, k_front<512>, wgs, dim3(nt), plan.lds, dd, tickets, np);
+        else if (nt <= 768) X2G_LAUNCH(ctx, k_front<768>, wgs, dim3(nt), plan.lds, dd, tickets, np);
+        else X2G_LAUNCH(ctx, k_front<1024>, wgs, dim3(nt), plan.lds, dd, tickets, np);
+        ++ctx->counts[X2G_COUNT_FRONT];
+        X2G_LAUNCH(ctx, k_front_out, dim3(bx, np), dim3(256), 0, dd);
+        X2G_HIP(hipGetLastError());
+    }
     return stats_end(ctx, ea, eb, plan.bytes * plan.nsweeps, 0, plan.nsweeps);
 }
 

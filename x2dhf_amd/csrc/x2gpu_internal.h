@@ -31,6 +31,8 @@ void set_error(const char *fmt, ...);
         }                                                                               \
     } while (0)
 
+constexpr size_t kMaxLds = 160 * 1024;   // LDS of a gfx950 compute unit
+
 // Growable device workspace owned by a context (never freed while a launch
 // that uses it may still run: growth synchronises the stream first).
 struct Workspace {

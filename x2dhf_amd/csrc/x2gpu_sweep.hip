@@ -3631,12 +3631,23 @@ extern "C" int x2g_call_counts(x2g_ctx *ctx, long long *out, int n)
 {
     X2G_CHECK(ctx && out && n >= 0, "x2g_call_counts: null argument");
     for (int k = 0; k < n; ++k) out[k] = k < X2G_COUNTS ? ctx->counts[k] : 0;
+    if (n > X2G_COUNT_WORKSPACE)
+        out[X2G_COUNT_WORKSPACE] = (long long)(ctx->ws[0].bytes + ctx->ws[3].bytes + ctx->ws[4].bytes);
     return X2G_OK;
 }
 
-extern "C" long long x2g_relax_workspace_bytes(int nni, int nmu, int prec)
+extern "C" long long x2g_relax_scheme_workspace_bytes(int nni, int nmu, int prec, int method, int ordering)
 {
     if (nni < 7 || nmu < 11 || (prec != 0 && prec != 1)) return -1;
+    if (method < X2G_MCSOR || method > X2G_SOR_BACKWARD || ordering < X2G_ORDER_COLWISE ||
+        ordering > X2G_ORDER_MIDDLE2)
+        return -1;
+    if (method != X2G_MCSOR || ordering != X2G_ORDER_COLWISE) {
+        // one padded array, relaxed in place, and the arrays by level of fronts
+        if (prec) return -1;
+        return (long long)(align256((size_t)(nni + 8) * (nmu + 8) * sizeof(double)) +
+                           front_workspace_bytes(nni, nmu, method, ordering));
+    }
     // the sizes x2g_relax_batch reserves per item, with the widest row
     // stride any sweep kind uses (nni+8 rounded up to 16 bytes, plus 16)
     const size_t elem = prec ? sizeof(float) : sizeof(double);
@@ -3645,6 +3656,15 @@ extern "C" long long x2g_relax_workspace_bytes(int nni, int nmu, int prec)
     const size_t n = (size_t)nni * nmu, ns = (size_t)split_size(nni, nmu);
     if (prec == 0) return (long long)(2 * pad + align256(2 * ns * sizeof(double)));
     return (long long)(2 * pad + 2 * align256(std::max(n, ns) * sizeof(float)));
+}
+
+extern "C" long long x2g_relax_workspace_bytes(int nni, int nmu, int prec)
+{
+    long long most = -1;
+    for (int m = X2G_MCSOR; m <= X2G_SOR_BACKWARD; ++m)
+        for (int o = X2G_ORDER_COLWISE; o <= X2G_ORDER_MIDDLE2; ++o)
+            most = std::max(most, x2g_relax_scheme_workspace_bytes(nni, nmu, prec, m, o));
+    return most;
 }
 
 extern "C" int x2g_residual_norms(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_relax_item *items, int n,

@@ -131,14 +131,15 @@ contains
   end function x2f_spec_bytes
 
   ! Device workspace bytes a job of this specification adds to its context
-  ! while it is relaxed (x2g_relax_workspace_bytes of its largest relaxation
-  ! call, the potentials, plus the padded copies of the batched quadratures
-  ! and their partial sums), without creating it; -1 as x2f_spec_bytes.
+  ! while it is relaxed (x2g_relax_scheme_workspace_bytes of its potentials and
+  ! of its orbitals, which are relaxed in calls of their own, plus the partial
+  ! sums of the batched quadratures), without creating it; -1 as
+  ! x2f_spec_bytes.
   integer(c_long_long) function x2f_spec_workspace_bytes(spec) bind(c, name='x2f_spec_workspace_bytes')
     type(x2f_spec), intent(in) :: spec
     type(case_t) :: c
     integer :: i, ierr, npotall
-    integer(c_long_long) :: per, npad
+    integer(c_long_long) :: pot, orb, relax
     x2f_spec_workspace_bytes = -1
     if (x2f_spec_bytes(spec) < 0) return
     c = case_t()
@@ -150,11 +151,27 @@ contains
     ierr = case_setup(c)
     if (ierr /= 0) return
     npotall = sum(c%npot(1:c%norb))
-    per = x2g_relax_workspace_bytes(spec%nni, spec%nmu, spec%prec)
-    if (per < 0) return
-    npad = int(spec%nni + 8, c_long_long)*int(spec%nmu + 8, c_long_long)
-    x2f_spec_workspace_bytes = int(max(npotall, int(spec%norb)), c_long_long)*per + &
-         int(spec%norb, c_long_long)*(8_c_long_long*npad + 65536_c_long_long)
+    pot = per_item(spec%pot_method)
+    orb = per_item(spec%orb_method)
+    if (pot < 0 .or. orb < 0) return
+    if (pot == orb) then
+       relax = int(max(npotall, int(spec%norb)), c_long_long)*pot
+    else   ! schemes that hold different buffers
+       relax = int(npotall, c_long_long)*pot + int(spec%norb, c_long_long)*orb
+    endif
+    x2f_spec_workspace_bytes = relax + int(spec%norb, c_long_long)*65536_c_long_long
+  contains
+    ! of one item, its scheme as set_scheme sets it
+    integer(c_long_long) function per_item(method)
+      integer(c_int), intent(in) :: method
+      if (spec%prec /= 0) then
+         per_item = x2g_relax_scheme_workspace_bytes(spec%nni, spec%nmu, spec%prec, 0_c_int, 0_c_int)
+         return
+      endif
+      per_item = x2g_relax_scheme_workspace_bytes(spec%nni, spec%nmu, spec%prec, method, spec%ordering)
+      if (per_item >= 0 .and. method == 1 .and. spec%alt_sweeps /= 0) per_item = max(per_item, &
+           x2g_relax_scheme_workspace_bytes(spec%nni, spec%nmu, spec%prec, 2_c_int, spec%ordering))
+    end function per_item
   end function x2f_spec_workspace_bytes
 
   ! The SCF loop's host bookkeeping (energy_change, convergence_control) fed

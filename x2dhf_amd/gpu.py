@@ -95,8 +95,8 @@ class ScfCtrl(C.Structure):
                 ("mm_due", _int), ("prec", _int), ("polish_end", _int), ("stopcode", _int), ("stop", _int)]
 
 
-# X2G_COUNT_*: bytes of descriptors staged, then launches by kernel
-COUNTS = ("staged", "phase", "strip", "sweep64", "sweep32", "chain", "resident", "front", "levels")
+# X2G_COUNT_*: bytes of descriptors staged, launches by kernel, bytes of workspace held
+COUNTS = ("staged", "phase", "strip", "sweep64", "sweep32", "chain", "resident", "front", "levels", "workspace")
 
 # name -> (restype, argtypes)
 _PROTOS = {
@@ -138,6 +138,7 @@ _PROTOS = {
     "x2g_relax_batch": (_int, [_vp, _vp, C.POINTER(RelaxItem), _int, _int, _int]),
     "x2g_residual_norms": (_int, [_vp, _vp, C.POINTER(RelaxItem), _int, _vp]),
     "x2g_relax_workspace_bytes": (C.c_longlong, [_int, _int, _int]),
+    "x2g_relax_scheme_workspace_bytes": (C.c_longlong, [_int] * 5),
     "x2g_lincomb": (_int, [_vp, _vp, _vp, _dbl, C.POINTER(Term), _int]),
     "x2g_wdot": (_int, [_vp, C.POINTER(Dot), _int, _vp]),
     "x2g_oneel": (_int, [_vp, _vp, _vp, _int, _int, _vp]),

@@ -201,3 +201,34 @@ def test_level_tables_beyond_one_pipeline(nni, nmu, method, name):
         assert ran.kernels == {"levels"}
         assert np.array_equal(w.get(), want), relerr(w.get(), want)
         g.destroy()
+
+
+def test_ordered_call_keeps_the_graphs_of_others():
+    """An ordered call that first reserves the workspace of fronts: the graph of
+    a colour-sweep call, which does not address it, is replayed as before."""
+    from x2dhf_amd import gpu
+    res = {}
+    for graphs in (0, 1):
+        with gpu.Context(0) as ctx:
+            p = Problems(ctx, [(169, 241, 3, 0, 0, 0)])
+            q = Problems(ctx, [(91, 121, 1, 0, 1, 1)])
+            gpu.check(ctx.lib.x2g_set_graphs(ctx.h, graphs))
+            c, r, out = gpu.C.c_longlong(), gpu.C.c_longlong(), []
+            print(f"graphs={graphs}", flush=True)
+            for call in range(4):
+                p.relax(1, 4)
+                ctx.sync()
+            gpu.check(ctx.lib.x2g_graph_counts(ctx.h, c, r))
+            before = c.value, r.value
+            q.relax(1, 4)
+            for call in range(3):
+                p.relax(1, 4)
+                ctx.sync()
+                out.append(p.get())
+            gpu.check(ctx.lib.x2g_graph_counts(ctx.h, c, r))
+            assert (c.value - before[0], r.value - before[1]) == (0, 3 * graphs)
+            res[graphs] = out
+            p.close()
+            q.close()
+    for a, b in zip(res[0], res[1]):
+        assert np.array_equal(a, b)

@@ -3478,7 +3478,10 @@ static std::string relax_signature(x2g_ctx *ctx, x2g_grid *const *grids, const x
     put(g_plan_gen.load());
     put(ctx->ws[0].ptr);
     put(ctx->ws[3].ptr);
-    put(ctx->ws[4].ptr);
+    // (only ordered items address it: its growth leaves the other graphs valid)
+    bool any_ordered = false;
+    for (int i = 0; i < n; ++i) any_ordered = any_ordered || ordered(items[i]);
+    put(any_ordered ? ctx->ws[4].ptr : nullptr);
     for (int i = 0; i < n; ++i) {
         const x2g_relax_item &it = items[i];
         const x2g_grid *g = grids[it.grid_index];

@@ -75,13 +75,17 @@ void *x2g_ctx_stream(x2g_ctx *ctx);
 int x2g_mem_info(x2g_ctx *ctx, size_t *free_bytes, size_t *total_bytes);
 /* Time the sweep launches of this context with HIP events on its stream: one
  * event pair around each run of back-to-back sweeps (a relaxation's maxsor2
- * sweeps), counted as that many launches, so the average launch time includes
- * the launch-to-launch gaps (on != 0 starts and clears the counters, 0 stops). */
+ * sweeps), so the average launch time includes the launch-to-launch gaps
+ * (on != 0 starts and clears the counters, 0 stops). */
 int x2g_stats_enable(x2g_ctx *ctx, int on);
 /* out[6] = {launches, milliseconds, algorithmic bytes} of the FP64 sweeps,
- * then of the FP32 sweeps.  Algorithmic bytes per relaxed point and sweep:
- * 4 words (read u, write u, read lhs, read rhs). */
+ * then of the FP32 sweeps.  A kernel that runs several sweeps counts as the
+ * one launch it is (the colour passes of a sweep, and its parts by grid width,
+ * count as one).  Algorithmic bytes per relaxed point and launch: 4 words (read
+ * u, write u, read lhs, read rhs), 3 where the source is known to be zero. */
 int x2g_stats_get(x2g_ctx *ctx, double *out);
+/* The same of one relaxation kernel, X2G_COUNT_PHASE .. X2G_COUNT_LEVELS: out[3]. */
+int x2g_stats_kernel(x2g_ctx *ctx, int kernel, double *out);
 
 /* What the calls on this context did so far, out[X2G_COUNT_*] for the first n
  * counts (those past the last are 0): bytes of launch descriptors staged, and

@@ -232,3 +232,35 @@ def test_ordered_call_keeps_the_graphs_of_others():
             q.close()
     for a, b in zip(res[0], res[1]):
         assert np.array_equal(a, b)
+
+
+# (shape, kernel, words per point and launch beyond the first, launches of ten sweeps)
+@pytest.mark.parametrize("shape, kernel, per_launch", [
+    ((91, 121, 700, 1, 0, 0), "chain", False), ((91, 121, 10, 1, 0, 0), "sweep32", True),
+    ((169, 241, 2, 0, 0, 0), "sweep64", True), ((61, 91, 2, 0, 0, 0), "resident", False),
+    ((61, 91, 2, 0, 1, 1), "front", False), ((61, 91, 2, 0, 1, 2), "levels", False),
+    ((361, 61, 2, 0, 0, 0), "strip", True),
+])
+def test_statistics_count_what_ran(shape, kernel, per_launch):
+    """Launches and algorithmic bytes by kernel: a launch of several sweeps is
+    one launch that moves its arrays once, and the first sweep of an FP32
+    correction does not read its zero source."""
+    from x2dhf_amd import gpu
+    nni, nmu, count, prec = shape[:4]
+    sweeps, iters = 10, 2
+    with gpu.Context(0) as ctx:
+        p = Problems(ctx, [shape])
+        p.relax(1, sweeps)  # tunes the plan
+        gpu.check(ctx.lib.x2g_stats_enable(ctx.h, 1))
+        with Ran(ctx) as ran:
+            p.relax(iters, sweeps)
+        st, tot = ctx.kernel_stats(), (gpu._dbl * 6)()
+        gpu.check(ctx.lib.x2g_stats_get(ctx.h, tot))
+        gpu.check(ctx.lib.x2g_stats_enable(ctx.h, 0))
+        assert ran.kernels == set(st) == {kernel}
+        launches, ms, nbytes = st[kernel]
+        assert launches == ran.n[kernel] and (launches == iters * sweeps) == per_launch
+        word, points = (4, 8)[prec == 0], count * (nni - 2) * (nmu - 5)
+        assert nbytes == word * points * (4 * launches - prec * iters)
+        assert ms > 0 and tuple(tot[3 * prec:3 * prec + 3]) == (launches, ms, nbytes) and tot[3 * (1 - prec)] == 0
+        p.close()

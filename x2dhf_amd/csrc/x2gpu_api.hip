@@ -199,11 +199,11 @@ int stats_begin(x2g_ctx *ctx, hipEvent_t *a, hipEvent_t *b)
     return X2G_OK;
 }
 
-int stats_end(x2g_ctx *ctx, hipEvent_t a, hipEvent_t b, double bytes, int prec, int launches)
+int stats_end(x2g_ctx *ctx, hipEvent_t a, hipEvent_t b, double bytes, int prec, int kernel, int launches)
 {
     if (!ctx->stats_on || !a) return X2G_OK;
     X2G_HIP(hipEventRecord(b, ctx->stream));
-    ctx->pending.push_back({a, b, bytes, prec, launches});
+    ctx->pending.push_back({a, b, bytes, prec, kernel, launches});
     if (ctx->pending.size() >= 4096) return stats_flush(ctx);
     return X2G_OK;
 }
@@ -215,9 +215,10 @@ int stats_flush(x2g_ctx *ctx)
     for (auto &p : ctx->pending) {
         float ms = 0.0f;
         X2G_HIP(hipEventElapsedTime(&ms, p.a, p.b));
-        ctx->st_launch[p.prec] += p.launches;
-        ctx->st_ms[p.prec] += ms;
-        ctx->st_bytes[p.prec] += p.bytes;
+        auto &st = ctx->stat[p.prec][p.kernel];
+        st.launches += p.launches;
+        st.ms += ms;
+        st.bytes += p.bytes;
         ctx->ev_pool.push_back(p.a);
         ctx->ev_pool.push_back(p.b);
     }
@@ -235,7 +236,8 @@ extern "C" int x2g_stats_enable(x2g_ctx *ctx, int on)
     int rc = stats_flush(ctx);
     if (rc) return rc;
     ctx->stats_on = on != 0;
-    for (int k = 0; k < 2; ++k) ctx->st_launch[k] = ctx->st_ms[k] = ctx->st_bytes[k] = 0;
+    for (auto &by_kernel : ctx->stat)
+        for (auto &st : by_kernel) st = {};
     return X2G_OK;
 }
 
@@ -245,9 +247,27 @@ extern "C" int x2g_stats_get(x2g_ctx *ctx, double *out)
     int rc = stats_flush(ctx);
     if (rc) return rc;
     for (int k = 0; k < 2; ++k) {
-        out[3 * k + 0] = ctx->st_launch[k];
-        out[3 * k + 1] = ctx->st_ms[k];
-        out[3 * k + 2] = ctx->st_bytes[k];
+        out[3 * k] = out[3 * k + 1] = out[3 * k + 2] = 0;
+        for (auto &st : ctx->stat[k]) {
+            out[3 * k + 0] += st.launches;
+            out[3 * k + 1] += st.ms;
+            out[3 * k + 2] += st.bytes;
+        }
+    }
+    return X2G_OK;
+}
+
+extern "C" int x2g_stats_kernel(x2g_ctx *ctx, int kernel, double *out)
+{
+    X2G_CHECK(ctx && out, "x2g_stats_kernel: null argument");
+    X2G_CHECK(kernel >= X2G_COUNT_PHASE && kernel <= X2G_COUNT_LEVELS, "x2g_stats_kernel: kernel %d", kernel);
+    int rc = stats_flush(ctx);
+    if (rc) return rc;
+    out[0] = out[1] = out[2] = 0;
+    for (auto &by_kernel : ctx->stat) {
+        out[0] += by_kernel[kernel].launches;
+        out[1] += by_kernel[kernel].ms;
+        out[2] += by_kernel[kernel].bytes;
     }
     return X2G_OK;
 }

@@ -110,8 +110,7 @@ struct ChainPlan {
     };
     std::vector<Chunk> chunks;
     std::vector<ChainOut> out;   // by problem
-    double bytes = 0;          // algorithmic bytes of all sweeps
-    int nsweeps = 0;
+    double bytes = 0;          // algorithmic bytes of all launches
 };
 // Plan nsweeps sweeps of the problems and stage the launch descriptors.
 int chain_plan(x2g_ctx *ctx, const std::vector<ChainProblem> &probs, int nsweeps, const ChainCut &cut,

@@ -160,12 +160,14 @@ bool chain_pays(x2g_ctx *ctx, const std::vector<ChainProblem> &probs, int nsweep
 int chain_plan(x2g_ctx *ctx, const std::vector<ChainProblem> &probs, int nsweeps, const ChainCut &cut, ChainPlan &plan)
 {
     plan.chunks.clear();
-    plan.nsweeps = nsweeps;
-    plan.bytes = 0;
-    for (auto &p : probs) plan.bytes += 4.0 * sizeof(float) * (double)(p.g->nni - 2) * (p.g->nmu - 5) * nsweeps;
     std::vector<ChainClass> cls = chain_classes(probs);
     for (auto &c : cls) X2G_CHECK(c.pack(cut.sweeps) && c.fit(cut.sweeps, cut.steps), "chain_plan: cut");
     const int nch = (nsweeps + cut.sweeps - 1) / cut.sweeps;
+    // a launch reads u and the pairs and writes u once, however many sweeps it
+    // runs; the first takes a zero u without reading it
+    plan.bytes = 0;
+    for (auto &p : probs)
+        plan.bytes += (4.0 * nch - (p.in ? 0.0 : 1.0)) * sizeof(float) * (double)(p.g->nni - 2) * (p.g->nmu - 5);
     plan.out.resize(probs.size());
     int done = 0;
     // Launches of one direction and length have the same descriptors, which are
@@ -255,7 +257,7 @@ int chain_run(x2g_ctx *ctx, const ChainPlan &plan)
         if ((rc = chain_kernel(ctx, c.packs, c.segs, c.wgs, c.nwg, c.sweeps, first ? 1 : 0))) return rc;
         first = false;
     }
-    return stats_end(ctx, ea, eb, plan.bytes, 1, plan.nsweeps);
+    return stats_end(ctx, ea, eb, plan.bytes, 1, X2G_COUNT_CHAIN, (int)plan.chunks.size());
 }
 
 }  // namespace x2g

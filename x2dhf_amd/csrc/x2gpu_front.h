@@ -27,7 +27,7 @@ struct FrontPlan {
     const FrontDesc *descs = nullptr;
     int n = 0, nsweeps = 0, threads = 0, most = 0;   // most: elements of the longest array by level
     size_t lds = 0;
-    double bytes = 0;          // algorithmic, of one sweep
+    double bytes = 0;          // algorithmic, of a launch: the arrays once, however many sweeps
 };
 int plan_fronts(x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps, FrontPlan &plan);
 // The sweeps.  Stages nothing, so it can run any number of times in a call.

@@ -513,7 +513,8 @@ int launch_fronts(x2g_ctx *ctx, const FrontPlan &plan)
         X2G_LAUNCH(ctx, k_front_out, dim3(bx, np), dim3(256), 0, dd);
         X2G_HIP(hipGetLastError());
     }
-    return stats_end(ctx, ea, eb, plan.bytes * plan.nsweeps, 0, plan.nsweeps);
+    const int launches = (plan.nsweeps + kFrontSweeps - 1) / kFrontSweeps;
+    return stats_end(ctx, ea, eb, plan.bytes * launches, 0, X2G_COUNT_FRONT, launches);
 }
 
 }  // namespace x2g

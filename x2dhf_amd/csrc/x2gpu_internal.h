@@ -65,9 +65,10 @@ struct x2g_ctx {
     // pending list is long
     bool stats_on = false;
     std::vector<hipEvent_t> ev_pool;
-    struct Pending { hipEvent_t a, b; double bytes; int prec, launches; };
+    struct Pending { hipEvent_t a, b; double bytes; int prec, kernel, launches; };
     std::vector<Pending> pending;
-    double st_launch[2] = {0, 0}, st_ms[2] = {0, 0}, st_bytes[2] = {0, 0};
+    struct Stat { double launches = 0, ms = 0, bytes = 0; };
+    Stat stat[2][X2G_COUNTS];      // by precision (1: FP32) and kernel (X2G_COUNT_*)
     long long counts[X2G_COUNTS] = {};  // x2g_call_counts
     // device blocks of x2g_malloc: sizes of the live ones, and freed ones
     // kept for reuse by size (all work on them is ordered by `stream`)
@@ -246,6 +247,6 @@ int pinned_out_reserve(x2g_ctx *ctx, size_t bytes);
 int scratch_init(x2g_ctx *ctx);
 // Sweep timing hooks (no-ops unless statistics are enabled on the context).
 int stats_begin(x2g_ctx *ctx, hipEvent_t *a, hipEvent_t *b);
-int stats_end(x2g_ctx *ctx, hipEvent_t a, hipEvent_t b, double bytes, int prec, int launches = 1);
+int stats_end(x2g_ctx *ctx, hipEvent_t a, hipEvent_t b, double bytes, int prec, int kernel, int launches);
 int stats_flush(x2g_ctx *ctx);
 }  // namespace x2g

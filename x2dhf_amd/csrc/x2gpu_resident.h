@@ -20,7 +20,7 @@ struct ResidentPlan {
     const ResidentDesc *descs = nullptr;
     int n = 0, groups = 1, threads = 64;
     size_t lds = 0;
-    double bytes = 0;          // algorithmic, of one sweep
+    double bytes = 0;          // algorithmic: the grids and pairs once, however many sweeps
 };
 int plan_resident(x2g_ctx *ctx, std::vector<ResidentDesc> &v, ResidentPlan &plan);
 // nsweeps sweeps of every problem.  Stages nothing, so it can run any number

@@ -197,7 +197,7 @@ int launch_resident(x2g_ctx *ctx, const ResidentPlan &plan, int nsweeps)
     }
     ++ctx->counts[X2G_COUNT_RESIDENT];
     X2G_HIP(hipGetLastError());
-    return stats_end(ctx, ea, eb, plan.bytes * nsweeps, 0, nsweeps);
+    return stats_end(ctx, ea, eb, plan.bytes, 0, X2G_COUNT_RESIDENT, 1);
 }
 
 }  // namespace x2g

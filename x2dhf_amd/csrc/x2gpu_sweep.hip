@@ -1949,7 +1949,11 @@ static int launch_sweeps(x2g_ctx *ctx, const SweepDesc<T> *de, const SweepDesc<T
         if ((rc = launch_sweep_once<T>(ctx, ev ? de : dodd, ev ? plan.even : plan.odd, plan, zsrc))) return rc;
         total += zsrc ? 0.75 * bytes : bytes;  // a zero source is not read: 3 words per point
     }
-    return stats_end(ctx, ea, eb, total, prec, nsweeps);
+    const int kernel = plan.kind == 0   ? X2G_COUNT_PHASE
+                       : plan.kind == 1 ? X2G_COUNT_STRIP
+                       : prec           ? X2G_COUNT_SWEEP32
+                                        : X2G_COUNT_SWEEP64;
+    return stats_end(ctx, ea, eb, total, prec, kernel, nsweeps);
 }
 
 static std::mutex g_attr_mutex;
@@ -2714,7 +2718,7 @@ static int launch_levels(x2g_ctx *ctx, const LevelDesc *dd, const std::vector<Le
     int rc = stage_flush(ctx);
     if (rc) return rc;
     double bytes = 0.0;
-    for (auto &d : v) bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5) * nsweeps;
+    for (auto &d : v) bytes += 32.0 * (double)(d.nni - 2) * (double)(d.nmu - 5);
     hipEvent_t ea, eb;
     if ((rc = stats_begin(ctx, &ea, &eb))) return rc;
     if (levels_pipe())
@@ -2723,7 +2727,7 @@ static int launch_levels(x2g_ctx *ctx, const LevelDesc *dd, const std::vector<Le
         X2G_LAUNCH(ctx, k_levels, dim3((int)v.size()), dim3(kLevelThreads), 0, dd, nsweeps);
     ++ctx->counts[X2G_COUNT_LEVELS];
     X2G_HIP(hipGetLastError());
-    return stats_end(ctx, ea, eb, bytes, 0, nsweeps);
+    return stats_end(ctx, ea, eb, bytes, 0, X2G_COUNT_LEVELS, 1);
 }
 
 // ---------------------------------------------------------------------------

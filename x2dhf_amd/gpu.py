@@ -109,6 +109,7 @@ _PROTOS = {
     "x2g_mem_info": (_int, [_vp, C.POINTER(_szt), C.POINTER(_szt)]),
     "x2g_stats_enable": (_int, [_vp, _int]),
     "x2g_stats_get": (_int, [_vp, _vp]),
+    "x2g_stats_kernel": (_int, [_vp, _int, _vp]),
     "x2g_call_counts": (_int, [_vp, C.POINTER(C.c_longlong), _int]),
     "x2g_malloc": (_int, [_vp, _szt, C.POINTER(_vp)]),
     "x2g_free": (_int, [_vp, _vp]),
@@ -226,6 +227,17 @@ class Context:
         out = (C.c_longlong * len(COUNTS))()
         check(self.lib.x2g_call_counts(self.h, out, len(COUNTS)))
         return dict(zip(COUNTS, out))
+
+    def kernel_stats(self):
+        """x2g_stats_kernel: {kernel: (launches, ms, algorithmic bytes)} of
+        those that ran since x2g_stats_enable."""
+        res, out = {}, (_dbl * 3)()
+        for k, name in enumerate(COUNTS[:-1]):
+            if k:
+                check(self.lib.x2g_stats_kernel(self.h, k, out))
+                if out[0]:
+                    res[name] = tuple(out)
+        return res
 
     def sync(self):
         check(self.lib.x2g_ctx_sync(self.h))

@@ -48,16 +48,18 @@ DECK = os.path.join(HERE, "tests", "golden", "decks", "config2_n2_331x601.data")
 GOLDEN = os.path.join(HERE, "tests", "golden", "scf_config2_n2_331x601.json")
 REF_EXE = os.path.join(HERE, "oracle", "_ref", "x2dhf_omp")
 TRAFFIC = os.path.join(HERE, "profiles", "traffic_sweep_n2_331x601.json")
-# the stream's dominant sweep launches: 2-row blocks of ring stride 528
 TRAFFIC_STREAM = os.path.join(HERE, "profiles", "traffic_sweep_stream_mix.json")
 # jobs the stream's server steps together (32 measured 3% faster than 16 on
 # the default stream; 64 the same as 32)
 STREAM_SLOTS = 32
 # problems of the stream traffic probe: (nni, nmu, count), a mix of the
-# stream's grid classes whose relaxed points (24.6 M, 394 MB of algorithmic
-# bytes per FP32 sweep) match the stream's average sweep launch
+# stream's grid classes (24.6 M relaxed points, 394 MB of algorithmic bytes per
+# FP32 launch)
 STREAM_PROBE = ((505, 901, 28), (409, 721, 20), (361, 601, 20), (217, 361, 16), (169, 241, 16))
 HBM_PEAK_GBS = 8000.0
+# the kernels behind the library's launch counts
+KERNELS = {"phase": "k_phase", "strip": "k_strip", "sweep64": "k_sweep<double>", "sweep32": "k_sweep<float>",
+           "chain": "k_chain_f32", "resident": "k_resident", "front": "k_front", "levels": "k_levels"}
 METRIC = "converged SCF solves/hr + p50/p99 latency vs plain FP64 GPU at ΔE<1e-8 Eh; GB/s"
 
 
@@ -90,8 +92,9 @@ def parse():
     ap.add_argument("--seed", type=int, default=0, help="poisson / stream: seed of the synthetic workload")
     ap.add_argument("--traffic-probe", nargs="?", const="n2", choices=["n2", "stream"],
                     help="only run a copy kernel of known size and a few sweeps (for rocprofv3 --pmc): n2 = "
-                         "--batch x 22 N2 331x601 potentials (FP32 and FP64), stream = the stream's widest "
-                         "launch class (12 problems on 505x901 and 12 on 361x601, FP32, 2-row blocks)")
+                         "--batch x 22 N2 331x601 potentials (FP32 and FP64), stream = a "
+                         "mix of the stream's grids (100 FP32 problems), as the library runs it and with one "
+                         "launch per sweep")
     ap.add_argument("--traffic-summary", nargs=2, metavar=("FETCH_CSV", "WRITE_CSV"),
                     help="turn the counter_collection.csv files of the FETCH_SIZE and WRITE_SIZE runs of "
                          "--traffic-probe into the per-launch HBM traffic file read by the benchmark")
@@ -153,9 +156,10 @@ def cpu_baseline(total_iters, iters):
 def traffic_probe(batch):
     """For the rocprofv3 counter runs: a copy kernel of known size (x2g_lincomb
     out = 1.0*a on a 1201 x 1201 grid: 11.5 MB read + 11.5 MB written per
-    launch, three launches), then one relaxation call (5 sweeps) in FP32 and
+    launch, three launches), then one relaxation call (10 sweeps) in FP32 and
     one in FP64 of --batch x 22 potentials on N2 331x601 grids: the sweep
-    launches of --batch jobs' potential relaxation in the benchmark."""
+    launches of --batch jobs' potential relaxation in the benchmark, by
+    whichever kernel runs them."""
     import numpy as np
     from x2dhf_amd import gpu, scf
     ctx = gpu.Context(0)
@@ -179,10 +183,10 @@ def traffic_probe(batch):
             keep += [f, r]
             items.append(gpu.RelaxItem(f.ptr, lhs.ptr, r.ptr, None, 1.9, 1, 1, 1, q))
     n = len(items)
-    gpu.check(ctx.lib.x2g_relax_batch(ctx.h, gh, (gpu.RelaxItem * n)(*items), n, 1, 5))
+    gpu.check(ctx.lib.x2g_relax_batch(ctx.h, gh, (gpu.RelaxItem * n)(*items), n, 1, 10))
     for it in items:
         it.prec = 0
-    gpu.check(ctx.lib.x2g_relax_batch(ctx.h, gh, (gpu.RelaxItem * n)(*items), n, 1, 5))
+    gpu.check(ctx.lib.x2g_relax_batch(ctx.h, gh, (gpu.RelaxItem * n)(*items), n, 1, 10))
     gpu.check(ctx.lib.x2g_ctx_sync(ctx.h))
     for g in gs:
         g.destroy()
@@ -193,15 +197,15 @@ def traffic_probe(batch):
 
 def traffic_probe_stream():
     """For the rocprofv3 counter runs: the copy kernel of traffic_probe, then
-    one relaxation call (5 FP32 sweeps) of the problems of STREAM_PROBE in one
-    batch, with the stream's usual plan for this class fixed (2-row blocks,
-    as many workgroups per CU as the LDS holds; no autotuning launches)."""
+    two relaxation calls of 10 FP32 sweeps of the problems of STREAM_PROBE in
+    one batch: as the library chooses, and with the plan that smaller batches
+    of this class use fixed (2-row blocks, as many workgroups per CU as the LDS
+    holds, one launch per sweep; no autotuning launches)."""
     import numpy as np
     from x2dhf_amd import gpu, scf
     ctx = gpu.Context(0)
     lib = ctx.lib
     gpu.check(lib.x2g_set_autotune(0))
-    gpu.check(lib.x2g_set_sweep_plan(2, 0, 0))
     rng = np.random.default_rng(0)
     cb = scf.grid_build(1201, 1201, 7.0, 7.0, 2.068, 40.0)
     big = gpu.Grid(ctx, 1201, 1201, *cb)
@@ -223,7 +227,9 @@ def traffic_probe_stream():
         gs.append(g)
     gh = (gpu._vp * len(gs))(*[g.h.value for g in gs])
     n = len(items)
-    gpu.check(lib.x2g_relax_batch(ctx.h, gh, (gpu.RelaxItem * n)(*items), n, 1, 5))
+    gpu.check(lib.x2g_relax_batch(ctx.h, gh, (gpu.RelaxItem * n)(*items), n, 1, 10))
+    gpu.check(lib.x2g_set_sweep_plan(2, 0, 0))
+    gpu.check(lib.x2g_relax_batch(ctx.h, gh, (gpu.RelaxItem * n)(*items), n, 1, 10))
     gpu.check(lib.x2g_ctx_sync(ctx.h))
     for g in gs:
         g.destroy()
@@ -233,93 +239,90 @@ def traffic_probe_stream():
     print("traffic probe done", flush=True)
 
 
-def traffic_summary_stream(fetch_csv, write_csv):
-    """HBM bytes per sweep launch of traffic_probe_stream, as traffic_summary:
-    counters scaled by the copy kernel, averaged over the four FP32 sweeps
-    that read their source (the first takes its zero start)."""
-    import csv
-    n_copy = 1201 * 1201 * 8
-
-    def per_kernel(path):
-        rows = sorted(csv.DictReader(open(path)), key=lambda r: int(r["Dispatch_Id"]))
-
-        def named(r, k):
-            n = r["Kernel_Name"]
-            return n.startswith(k) or f"::{k}(" in n or f"::{k}<" in n
-
-        copy = [float(r["Counter_Value"]) * 1024 for r in rows if named(r, "k_lincomb")]
-        sweep = [float(r["Counter_Value"]) * 1024 for r in rows if named(r, "k_sweep")]
-        if len(copy) != 3 or len(sweep) != 5:
-            raise SystemExit(f"{path}: expected 3 copy and 5 sweep dispatches, found {len(copy)} and {len(sweep)}")
-        return sum(copy) / len(copy), sweep[1:]
-
-    fc, fv = per_kernel(fetch_csv)
-    wc, wv = per_kernel(write_csv)
-    kf, kw = n_copy / fc, n_copy / wc
-    algo = sum(16.0 * cnt * (nni - 2) * (nmu - 5) for nni, nmu, cnt in STREAM_PROBE)
-    rd, wr = kf * sum(fv) / len(fv), kw * sum(wv) / len(wv)
-    out = {"workload": " + ".join(f"{cnt} x {nni}x{nmu}" for nni, nmu, cnt in STREAM_PROBE) +
-           " FP32 correction problems, one k_sweep<float,1,528,2> launch", "fetch_factor": kf, "write_factor": kw,
-           "fp32": {"hbm_read_bytes": rd, "hbm_write_bytes": wr, "hbm_bytes_per_launch": rd + wr,
-                    "algorithmic_bytes_per_launch": algo, "traffic_over_algorithmic": (rd + wr) / algo}}
-    with open(TRAFFIC_STREAM, "w") as f:
-        json.dump(out, f, indent=1)
-    print(json.dumps(out, indent=1))
-
-
-def traffic_summary(fetch_csv, write_csv, batch):
-    """HBM bytes per sweep launch from the rocprofv3 FETCH_SIZE / WRITE_SIZE
-    runs of --traffic-probe.  Each counter (KiB per dispatch) is scaled by
-    what it reads for the probe's copy kernel (x2g_lincomb, bytes known), and
-    averaged over the probe's FP32 sweep launches that read their source
-    (launches 2-5: the first sweep of a correction takes its zero start
-    without reading it) and its FP64 launches (the last five)."""
+def traffic_summary(fetch_csv, write_csv, probe, batch):
+    """HBM bytes per sweep launch of a traffic probe, by kernel, from the
+    rocprofv3 FETCH_SIZE / WRITE_SIZE runs of --traffic-probe.  Each counter
+    (KiB per dispatch) is scaled by what it reads for the probe's copy kernel
+    (x2g_lincomb, bytes known), and averaged over a kernel's launches that read
+    their source (an FP32 correction's first launch takes its zero start
+    without reading it)."""
     import csv
     n_copy = 1201 * 1201 * 8  # bytes read and written by one copy launch
 
     def per_kernel(path):
         rows = sorted(csv.DictReader(open(path)), key=lambda r: int(r["Dispatch_Id"]))
         # kernel names come demangled ("x2g::k_lincomb(double*, ...)") or bare ("k_lincomb")
-        def named(r, k):
-            n = r["Kernel_Name"]
-            return n.startswith(k) or f"::{k}(" in n or f"::{k}<" in n
+        def values(kernel):
+            return [float(r["Counter_Value"]) * 1024 for r in rows
+                    if r["Kernel_Name"] == kernel or
+                    any(r["Kernel_Name"].startswith(kernel + e) or f"::{kernel}{e}" in r["Kernel_Name"]
+                        for e in ("(", "<", ","))]
 
-        copy = [float(r["Counter_Value"]) * 1024 for r in rows if named(r, "k_lincomb")]
-        sweep = [float(r["Counter_Value"]) * 1024 for r in rows if named(r, "k_sweep")]
-        if len(copy) != 3 or len(sweep) != 10:
-            raise SystemExit(f"{path}: expected 3 copy and 10 sweep dispatches, found {len(copy)} and {len(sweep)}")
-        return sum(copy) / len(copy), sweep[1:5], sweep[5:]
+        copy = values("k_lincomb")
+        runs = {"k_chain_f32": values("k_chain_f32")[1:], "k_sweep<float>": values("k_sweep<float")[1:],
+                "k_sweep<double>": values("k_sweep<double")}
+        runs = {k: v for k, v in runs.items() if v}
+        if len(copy) != 3 or not runs:
+            raise SystemExit(f"{path}: expected 3 copy and some sweep dispatches, found {len(copy)} and {list(runs)}")
+        return sum(copy) / len(copy), runs
 
-    fc, f32, f64 = per_kernel(fetch_csv)
-    wc, w32, w64 = per_kernel(write_csv)
+    fc, fetch = per_kernel(fetch_csv)
+    wc, write = per_kernel(write_csv)
+    if {k: len(v) for k, v in fetch.items()} != {k: len(v) for k, v in write.items()}:
+        raise SystemExit(f"{fetch_csv} and {write_csv} are not of the same probe")
     kf, kw = n_copy / fc, n_copy / wc  # counter -> bytes factors from the copy kernel
-    out = {"workload": f"{batch} x 22 potentials, N2 331x601, one sweep launch", "fetch_factor": kf,
-           "write_factor": kw}
-    algo = {4: 0.0, 8: 0.0}
-    for t in (4, 8):
-        algo[t] = batch * 22 * 4.0 * t * (331 - 2) * (601 - 5)
-    for key, fv, wv, t in (("fp32", f32, w32, 4), ("fp64", f64, w64, 8)):
-        rd = kf * sum(fv) / len(fv)
-        wr = kw * sum(wv) / len(wv)
-        out[key] = {"hbm_read_bytes": rd, "hbm_write_bytes": wr, "hbm_bytes_per_launch": rd + wr,
-                    "algorithmic_bytes_per_launch": algo[t], "traffic_over_algorithmic": (rd + wr) / algo[t]}
-    os.makedirs(os.path.dirname(TRAFFIC), exist_ok=True)
-    with open(TRAFFIC, "w") as f:
+    grids = STREAM_PROBE if probe == "stream" else ((331, 601, 22 * batch),)
+    points = sum(cnt * (nni - 2) * (nmu - 5) for nni, nmu, cnt in grids)
+    out = {"workload": " + ".join(f"{cnt} x {nni}x{nmu}" for nni, nmu, cnt in grids) + ", 10 sweeps",
+           "fetch_factor": kf, "write_factor": kw, "kernels": {}}
+    for k in fetch:
+        rd, wr = kf * sum(fetch[k]) / len(fetch[k]), kw * sum(write[k]) / len(write[k])
+        algo = 4.0 * (8 if "double" in k else 4) * points
+        out["kernels"][k] = {"launches": len(fetch[k]), "hbm_read_bytes": rd, "hbm_write_bytes": wr,
+                             "hbm_bytes_per_launch": rd + wr, "algorithmic_bytes_per_launch": algo,
+                             "traffic_over_algorithmic": (rd + wr) / algo}
+    path = TRAFFIC_STREAM if probe == "stream" else TRAFFIC
+    os.makedirs(os.path.dirname(path), exist_ok=True)
+    with open(path, "w") as f:
         json.dump(out, f, indent=1)
+        f.write("\n")
     print(json.dumps(out, indent=1))
 
 
-def sweep_roofline(st, prec):
-    """Roofline object of the sweep kernel of precision prec (1 FP32, 0 FP64)
-    from the library's HIP-event statistics [launches, ms, bytes] x 2."""
-    k = 1 if prec else 0
-    launches, ms, nbytes = st[3 * k], st[3 * k + 1], st[3 * k + 2]
+def add_stats(total, ctx):
+    """Add a context's sweep statistics {kernel: (launches, ms, bytes)}."""
+    for k, v in ctx.kernel_stats().items():
+        total[k] = tuple(a + b for a, b in zip(total.get(k, (0.0, 0.0, 0.0)), v))
+    return total
+
+
+def sweep_roofline(stats, traffic_file=None):
+    """Roofline object of the sweep kernel that took most of the time, from the
+    library's HIP-event statistics {kernel: (launches, ms, algorithmic bytes)};
+    traffic: its measured/algorithmic HBM bytes in traffic_file times this
+    run's algorithmic bytes per launch."""
+    if not stats:
+        return {"bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None, "traffic": None,
+                "kernel": None, "algorithmic_bytes_per_launch": None, "avg_launch_us": None, "launches": 0}
+    name = max(stats, key=lambda k: stats[k][1])
+    launches, ms, nbytes = stats[name]
     achieved = nbytes / (ms * 1e-3) / 1e9 if ms else None
-    return {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": None,
-            "kernel": "k_sweep<float>" if k else "k_sweep<double>",
-            "algorithmic_bytes_per_launch": nbytes / launches if launches else None,
-            "avg_launch_us": ms / launches * 1e3 if launches else None, "launches": launches}
+    roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": None, "kernel": KERNELS[name],
+            "algorithmic_bytes_per_launch": nbytes / launches, "avg_launch_us": ms / launches * 1e3,
+            "launches": int(launches),
+            "all_kernels": {KERNELS[k]: {"launches": int(n), "ms": t, "algorithmic_bytes": b}
+                            for k, (n, t, b) in sorted(stats.items())}}
+    if traffic_file and os.path.exists(traffic_file):
+        ratio = json.load(open(traffic_file)).get("kernels", {}).get(KERNELS[name], {}).get("traffic_over_algorithmic")
+        if ratio:
+            roof["traffic"] = ratio * nbytes / launches
+            roof["traffic_over_algorithmic"] = ratio
+            roof["traffic_source"] = ("measured/algorithmic HBM bytes of this kernel's launches in " +
+                                      os.path.relpath(traffic_file, HERE) + " (rocprofv3 FETCH_SIZE / WRITE_SIZE "
+                                      "runs of bench.py --traffic-probe) times this run's average algorithmic bytes "
+                                      "per launch")
+    return roof
 
 
 def bench_ordered(args):
@@ -382,7 +385,6 @@ def bench_poisson(args):
     from x2dhf_amd import poisson
     count = args.count or 256
     out = poisson.run(count=count, seed=args.seed, prec=args.prec, tol=1e-12)
-    st = out["stats"]
     sweeps = sum(out["calls"]) * 10
     line = {
         "metric": "converged synthetic Poisson solves/s (mixed grids, FP32 sweeps + FP64 residuals)",
@@ -399,7 +401,7 @@ def bench_poisson(args):
         "max_residual_over_fp64_floor": max(r / f for r, f in zip(out["residuals"], out["floors"]) if f > 0)
         if any(f > 0 for f in out["floors"]) else None,
         "setup_s": out["setup_s"], "problem_sweeps": sweeps,
-        "roofline": sweep_roofline(st, args.prec),
+        "roofline": sweep_roofline(out["kernel_stats"]),
         "cpu_baseline": None,
     }
     print(json.dumps(line), flush=True)
@@ -410,8 +412,7 @@ def serve_stream(reqs, prec, stats=False, graphs=False, groups=1):
     server at the given precision (graphs: relaxations replayed from captured
     HIP graphs; groups > 1: that many server groups on their own streams and
     host threads, serve.GroupServer); returns (handles, elapsed_s, sweep
-    stats summed over the groups' contexts)."""
-    import ctypes as C
+    stats by kernel summed over the groups' contexts)."""
     from x2dhf_amd import gpu, scf, serve
     if groups > 1:
         server = serve.GroupServer(groups=groups, max_active=STREAM_SLOTS, graphs=graphs)
@@ -433,12 +434,10 @@ def serve_stream(reqs, prec, stats=False, graphs=False, groups=1):
     for c in ctxs:
         gpu.check(lib.x2g_ctx_sync(c.h))
     elapsed = max(h.finished for h in handles) - t0
-    tot = [0.0] * 6
+    tot = {}
     if stats:
         for c in ctxs:
-            st = (C.c_double * 6)()
-            gpu.check(lib.x2g_stats_get(c.h, st))
-            tot = [a + b for a, b in zip(tot, st)]
+            add_stats(tot, c)
     server.close()
     return handles, elapsed, tot
 
@@ -530,14 +529,15 @@ def bench_stream(args):
     for w in range(args.warmup):
         serve_stream(serve.poisson_stream(min(8, count), args.rate, seed=1000 + w, prec=args.prec), args.prec)
         print(f"# warmup stream {w + 1} done", file=sys.stderr, flush=True)
-    timed, handles, elapsed, st = [], [], 0.0, [0.0] * 6
+    timed, handles, elapsed, st = [], [], 0.0, {}
     for k in range(args.steps):
         reqs = serve.poisson_stream(count, args.rate, seed=args.seed + k, prec=args.prec)
         h, e, s = serve_stream(reqs, args.prec, stats=True)
         timed += reqs
         handles += h
         elapsed += e
-        st = [a + b for a, b in zip(st, s)]
+        for q, v in s.items():
+            st[q] = tuple(a + b for a, b in zip(st.get(q, (0.0, 0.0, 0.0)), v))
         print(f"# timed stream {k + 1}: {count} requests in {e:.2f} s", file=sys.stderr, flush=True)
     conv = [h.result["stop"] for h in handles]
     ok = [serve.converged(h.result) for h in handles]
@@ -622,16 +622,7 @@ def bench_stream(args):
                  "max_abs_dE_vs_served": max(dEp) if dEp else None}
         print(f"# plain FP64 GPU, {n} requests one at a time: {plain_s:.2f} s, max |dE| {plain['max_abs_dE_vs_served']}",
               file=sys.stderr, flush=True)
-    roof = sweep_roofline(st, args.prec)
-    tfile = TRAFFIC_STREAM if args.prec else TRAFFIC
-    if os.path.exists(tfile) and roof.get("algorithmic_bytes_per_launch"):
-        ratio = json.load(open(tfile)).get("fp32" if args.prec else "fp64", {}).get("traffic_over_algorithmic")
-        if ratio:
-            roof["traffic"] = ratio * roof["algorithmic_bytes_per_launch"]
-            roof["traffic_source"] = ("measured/algorithmic HBM bytes of the probe launch in " +
-                                      os.path.relpath(tfile, HERE) + " (rocprofv3 FETCH_SIZE / WRITE_SIZE runs of "
-                                      "bench.py --traffic-probe) times this run's average algorithmic bytes per "
-                                      "launch")
+    roof = sweep_roofline(st, TRAFFIC_STREAM if args.prec else TRAFFIC)
     cpu = None if args.no_cpu else cpu_baseline_stream(timed, args.cpu_seconds)
     by_mol = {}
     for (t, name, spec), h in zip(timed, handles):
@@ -672,10 +663,7 @@ def bench_stream(args):
 def main():
     args = parse()
     if args.traffic_summary:
-        if args.probe == "stream":
-            traffic_summary_stream(*args.traffic_summary)
-        else:
-            traffic_summary(*args.traffic_summary, args.batch)
+        traffic_summary(*args.traffic_summary, args.probe, args.batch)
         return
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
@@ -697,7 +685,6 @@ def main():
     if args.workload == "ordered":
         bench_ordered(args)
         return
-    import ctypes as C
     from x2dhf_amd import gpu, serve
     E_ref = json.load(open(GOLDEN))["etot"]
     ref_iters = len(json.load(open(GOLDEN))["iterations"])
@@ -731,25 +718,12 @@ def main():
         print(f"# timed wave {s + 1} done", file=sys.stderr, flush=True)
     gpu.check(lib.x2g_ctx_sync(server.ctx.h))
     elapsed = time.perf_counter() - t0
-    st = (C.c_double * 6)()
-    gpu.check(lib.x2g_stats_get(server.ctx.h, st))
+    roof = sweep_roofline(add_stats({}, server.ctx), TRAFFIC)
     server.close()
 
     lat = [r.latency for r in timed]
     dE = max(abs(r.result["etot"] - E_ref) for r in timed)
     value = len(timed) / elapsed * 3600.0
-    k = 1 if st[4] >= st[1] else 0            # dominant sweep precision by time
-    launches, ms, nbytes = st[3 * k], st[3 * k + 1], st[3 * k + 2]
-    avg_us = ms / launches * 1e3 if launches else None
-    per_launch = nbytes / launches if launches else None
-    achieved = nbytes / (ms * 1e-3) / 1e9 if ms else None
-    # HBM traffic per launch: the ratio of measured to algorithmic bytes of the
-    # 352-potential launch (rocprofv3 counters on --traffic-probe, stored by
-    # --traffic-summary) applied to this run's average launch
-    traffic, ratio = None, None
-    if os.path.exists(TRAFFIC) and per_launch:
-        ratio = json.load(open(TRAFFIC)).get("fp32" if k == 1 else "fp64", {}).get("traffic_over_algorithmic")
-        traffic = ratio * per_launch if ratio else None
     cpu = None if args.no_cpu else cpu_baseline(ref_iters, [int(x) for x in args.cpu_iters.split(",")])
     line = {
         "metric": METRIC,
@@ -774,11 +748,7 @@ def main():
         "max_abs_dE_vs_fp64_oracle": dE,
         "plain_fp64_gpu": plain,
         "speedup_vs_plain_fp64_gpu": value / plain["solves_per_hr"] if plain else None,
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": traffic,
-                     "kernel": "k_sweep<float>" if k == 1 else "k_sweep<double>",
-                     "algorithmic_bytes_per_launch": per_launch, "avg_launch_us": avg_us,
-                     "launches": launches, "traffic_over_algorithmic": ratio},
+        "roofline": roof,
         "cpu_baseline": cpu,
     }
     print(json.dumps(line), flush=True)

@@ -196,9 +196,10 @@ def run(count=256, seed=0, prec=1, tol=1e-12, stall_checks=40):
     t2 = time.perf_counter()
     st = (C.c_double * 6)()
     gpu.check(b.lib.x2g_stats_get(b.ctx.h, st))
+    kernels = b.ctx.kernel_stats()
     gpu.check(b.lib.x2g_stats_enable(b.ctx.h, 0))
     ok, floors = b.solved(res, tol)
     b.close()
     return dict(problems=count, setup_s=t1 - t0, solve_s=t2 - t1, max_residual=float(res.max()),
                 solved=int(ok.sum()), at_tol=int((res <= tol).sum()), residuals=res.tolist(),
-                floors=floors.tolist(), calls=calls.tolist(), stats=list(st))
+                floors=floors.tolist(), calls=calls.tolist(), stats=list(st), kernel_stats=kernels)

@@ -80,3 +80,32 @@ def test_recorded_ratios_name_their_kernels():
         assert "k_chain_f32" in got["kernels"], path
         for k in got["kernels"].values():
             assert 0.5 < k["traffic_over_algorithmic"] < 4.0, path
+
+
+def test_a_step_is_a_share_of_one_stream(monkeypatch, capsys):
+    """Without --count the timed work is one stream, whatever the steps: 64
+    requests, or 4 a step; with it, a stream of that many per step.  Energies
+    compare equal where both servings of a request stopped on a NaN."""
+    from types import SimpleNamespace as Ns
+    nan = float("nan")
+    for steps, count, streams, per in ((1, None, 1, 64), (10, None, 1, 64), (20, None, 1, 80), (3, 5, 3, 5)):
+        sizes = []
+
+        def serve_stream(reqs, prec, stats=False, graphs=False, groups=1):
+            sizes.append(len(reqs))
+            res = [dict(stop="not a number", etot=nan) if k == 3 else
+                   dict(stop="orbital energy threshold", etot=-1.0 - k) for k in range(len(reqs))]
+            return [Ns(result=r, latency=1.0) for r in res], 2.0, {}
+
+        monkeypatch.setattr(bench, "serve_stream", serve_stream)
+        argv = ["bench.py", "--steps", str(steps), "--warmup", "2", "--no-cpu", "--no-plain"]
+        monkeypatch.setattr(sys, "argv", argv + (["--count", str(count)] if count else []))
+        bench.bench_stream(bench.parse())
+        line = json.loads(capsys.readouterr().out.strip().splitlines()[-1])
+        # two warm-up streams, then as served, in FP64, with graphs, in two groups
+        assert sizes[2:] == [per] * 4 * streams and max(sizes[:2]) <= 8
+        assert line["steps"] == steps and line["requests"] == streams * per
+        assert line["config"]["requests_per_step"] == streams * per / steps
+        assert line["ms_per_step"] == pytest.approx(2000.0 * streams / steps)
+        assert line["graph_replay"]["energies_identical_to_eager"]
+        assert line["two_groups_graph_replay"]["energies_identical_to_eager"]

@@ -158,15 +158,26 @@ const double *x2g_grid_suppl(x2g_grid *g, int k);
  * it fits, else 2, else 1; 1 = one launch per colour pass; 2 = the first
  * pipelined strip kernel (natural lhs/rhs; falls back to 1 for grids too wide
  * for its LDS ring).  strip_rows > 0 fixes the strip height (rounded up to a
- * multiple of 4), <= 0 lets the library choose. */
+ * multiple of 4), <= 0 lets the library choose.  With the default engine, a
+ * free strip height and a free plan (x2g_set_sweep_plan), the strip sweep gives
+ * way to kernels that run several sweeps per launch with the same result: FP64
+ * calls of small grids keep each on a compute unit for all sweeps, and large
+ * batches of FP32 corrections run in chains of sweeps. */
 int x2g_set_sweep_engine(int engine, int strip_rows);
 
 /* Schedule of ordered sweeps (x2g_relax_ordered, relax items with a method
  * other than the col-wise MCSOR) for all later calls of this process:
  * 1 = default: the sweeps pipelined, each a fixed number of dependency
- * levels behind the one before, one barrier per step of all of them;
- * 0 = one dependency level of one sweep per barrier (X2G_LEVELS=phase).
- * Both give the sequential routine's result bit for bit (sormcsor.F90:20-132,
+ * levels behind the one before.  SOR in orders that walk rows and columns
+ * straight, reversed or from the middle (not middlemt, nor backward from the
+ * middle) runs a workgroup per sweep and a thread per column, on grids of 24 x
+ * 24 points and more, up to 504 columns where the rows start in the middle and
+ * 1016 elsewhere (fewer where the other axis is long: a sweep's row weights lie
+ * in LDS); all else, and calls for whose arrays by level there is no memory, run
+ * a workgroup per problem on level tables, with one barrier per step of all
+ * sweeps.  0 = one dependency level of one sweep per barrier for all
+ * (X2G_LEVELS=phase).
+ * Each gives the sequential routine's result bit for bit (sormcsor.F90:20-132,
  * 143-386 with one thread).  No counterpart in the reference: a choice of
  * this library's schedule. */
 int x2g_set_levels_pipeline(int on);
@@ -176,19 +187,21 @@ int x2g_set_levels_pipeline(int on);
  * number of ring classes, total rows rounded to a power of sqrt 2) the
  * candidate k_sweep plans -- blocks of 4 or 2 rows, workgroups per CU 1, 2, 3
  * or as many as the LDS ring allows, one launch or one per ring class -- are
- * timed on that batch and the fastest is kept for the shape.  on = 0 / 1
+ * timed on that batch and the fastest is kept for the shape.  Batches that run
+ * resident or in chains (x2g_set_sweep_engine) are not tuned.  on = 0 / 1
  * turns it off / on, -1 forgets the tuned shapes.  No reference counterpart. */
 int x2g_set_autotune(int on);
 /* Fix the k_sweep plan for later calls of this process: block_rows 4 or 2
  * (0: 4), wg_per_cu workgroups per CU the segment planner fills (0: as many
  * as the LDS ring allows), split 1 = one launch per ring class.  Any nonzero
- * value keeps the autotuner out; (0, 0, 0) hands the choice back to it.  The
- * results do not depend on the plan.  No reference counterpart. */
+ * value keeps the autotuner out, and the kernels that run several sweeps per
+ * launch; (0, 0, 0) hands the choice back.  The results do not depend on the
+ * plan.  No reference counterpart. */
 int x2g_set_sweep_plan(int block_rows, int wg_per_cu, int split);
 /* Replay x2g_relax_batch from captured HIP graphs on this context (default
  * off; X2G_GRAPHS=1 at context creation turns it on).  The second call with
  * the same signature -- items, grids, sweep counts, sweep-plan settings and
- * workspace -- is captured into a graph of its kernel launches, with the
+ * the workspace it uses -- is captured into a graph of its kernel launches, with the
  * launch descriptors in a device arena of the graph's own; later calls with
  * that signature launch the graph.  Results are those of the eager calls.
  * Not while sweep statistics are on.  on = 0 releases the graphs.  No
@@ -233,9 +246,10 @@ int x2g_mcsor_noalloc(x2g_grid *g, int isym, int bkind, double *work_d, const do
  * (initCBAllocArrays.F90:2408-2810; the reference's default is middle) on the
  * padded work_d, in place: nsweeps sweeps, each followed by the boundary
  * lines.  The points are updated in exactly the reference's sequential order
- * of dependencies: each sweep runs as a list of phases of mutually
- * independent points (for sor: the anti-diagonals of the ordering's
- * (position in row, row) plane), all in one workgroup.  The orderings are
+ * of dependencies: each sweep runs as levels of mutually independent points
+ * (for sor: the anti-diagonals of the ordering's (position in row, row) plane),
+ * one workgroup per sweep or one for all (x2g_set_levels_pipeline).  The
+ * orderings are
  * the reference's `order` card values (read_order, inputInterface.F90:2397):
  * col-wise, middle, middlemt, row-wise, rrow-wis, test1, test2, test3,
  * test4, middle2.  Method X2G_SOR_BACKWARD is sor walking the ordering from
@@ -298,9 +312,13 @@ typedef struct {
     int ordering;
 } x2g_relax_item;
 
-/* Relax n problems, possibly on different grids, together: every sweep of
- * every problem is issued in one fused launch (items of another method or
- * ordering: all their sweeps in one launch, a workgroup per item). */
+/* Relax n problems, possibly on different grids, together: a launch takes one
+ * sweep of every problem, or several (x2g_set_sweep_engine); items of another
+ * method or ordering take all their sweeps in one launch, a workgroup per item
+ * and sweep or per item (x2g_set_levels_pipeline; a workgroup per sweep runs
+ * 1024 sweeps per launch at most, between launches that lay its arrays out and
+ * put them back).  What a call stages for its launches depends on its items
+ * only, not on the numbers of iterations and sweeps. */
 int x2g_relax_batch(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_relax_item *items, int n,
                     int maxsor1, int maxsor2);
 

@@ -18,11 +18,16 @@
 // A point's operations and their order are k_sweep's, so a result does not
 // depend on which of the two a batch's size chooses.
 //
-// Bound by instruction issue: a step is 165 VALU instructions per wave, two
-// waves share a SIMD, and a barrier ends it: 0.82 microseconds (0.95 where all
-// CUs stream), of them 0.18 the barrier.  Per sweep: 352 grids of 331 x 601
-// took 312 microseconds with one launch per sweep and take 183 in pairs of
-// sweeps; 104 grids of 169 x 241 .. 505 x 901 took 127 and take 103.
+// Bound by the length of a step, 168 VALU instructions per wave with two waves
+// on a SIMD and a barrier at its end, and where all CUs stream by memory as
+// well: pairs of sweeps over 352 grids of 331 x 601 are 390 steps in 389
+// microseconds that move 2.0 GB (5.2 TB/s), 1.8 times the arrays' size, as
+// every sweep of a launch reads the pairs and the segments' ends are read
+// twice.  Per sweep that is 195 microseconds, 315 with one launch per sweep;
+// 104 grids of 169 x 241 .. 505 x 901 take 110 and took 127.
+//
+// The 256 registers of a wave do not hold all: 14 are spilled, and their
+// scratch traffic counts with the loads that a first stage waits for.
 #pragma once
 #include "x2gpu_internal.h"
 #include <type_traits>
@@ -417,8 +422,9 @@ __device__ __forceinline__ void chain_stage(const ChainPack __attribute__((addre
     auto step = [&](auto uc) {
         constexpr int u = decltype(uc)::value, cur = u & 1, prev = cur ^ 1, c = BASE + u;   // c: row s
         if constexpr (FIRST) {
-            // row s + 5 is in: the pairs of kLead - 1 steps and kLead - 2 rows were
-            // issued after it
+            // row s + 5 is in: at least the pairs of kLead - 1 steps and kLead - 2
+            // rows were issued after it (spilled registers add to them, which only
+            // lengthens the wait: operations complete in order)
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NP * (kLead - 1) + kFetch * (kLead - 2)) : "memory");
             row_get(fin[(u + 5) % kRing], lane, win[c + 5]);
             if (fetch) fetch_row(s + 4 + kLead, (u + 4 + kLead) % kRing);

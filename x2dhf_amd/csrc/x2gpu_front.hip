@@ -23,8 +23,9 @@
 // The point update keeps the reference's expression and forms no fused
 // multiply-add: the result is the sequential one bit for bit.
 //
-// Bound by the latency of a step, 0.9 (169 x 241) to 1 microsecond (331 x 601),
-// and by the levels that must pass.  10 sweeps in the middle ordering against
+// Bound by the latency of a step, 0.9 (169 x 241) to 1 microsecond (331 x 601:
+// 803 microseconds for 10 sweeps, whose waves wait in 63 % of their cycles), and
+// by the levels that must pass.  10 sweeps in the middle ordering against
 // one workgroup on a level table: 331 x 601 12.6 -> 0.83 ms, three problems
 // of 169 x 241 2.65 -> 0.50 ms.  Blocks of 8 steps: 1.19 and 0.62 ms, as the
 // next sweep then follows further behind.

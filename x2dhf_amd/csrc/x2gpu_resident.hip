@@ -9,12 +9,16 @@
 // A thread's groups lie in one row, so its row weights stay in registers; the
 // (omega/lhs, rhs) pairs of a pass are loaded during the pass before.
 //
-// 10 sweeps of one 91 x 121 function through x2g_mcsor: 313 -> 112 microseconds.
-// A pass then takes 1.7 microseconds, bound by the LDS reads (17 values of
-// each of 2070 points) and the arithmetic of one compute unit.
+// 10 sweeps of one 91 x 121 function through x2g_mcsor: 313 -> 112 microseconds,
+// 106 of them the kernel: 50 passes and 20 boundary phases, bound by the LDS
+// reads (17 values of each of 2070 points a pass; waves wait for LDS in three
+// quarters of the cycles that an instruction waits) and the arithmetic of one
+// compute unit.  Four groups a thread spill 14 registers.
 //
 // The point and the boundary values are k_sweep's own, rounding for rounding,
-// so a problem's result does not depend on what else is in its batch.
+// so a problem's result does not depend on which of the two a batch's sizes
+// choose.  (Both end at 336 columns: one wider FP64 grid sends the whole batch
+// to k_strip or k_phase, which round differently.)
 #include "x2gpu_resident.h"
 #include <algorithm>
 

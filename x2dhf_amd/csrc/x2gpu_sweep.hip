@@ -412,12 +412,15 @@ __global__ void k_rhs_product(const ProdDesc *__restrict__ pd)
 
 // ---------------------------------------------------------------------------
 // k_sweep: the pipelined strip sweep (the block schedule of k_strip, with
-// blocks of BR = 4 or 2 rows) with a fixed lane -> work map.  Wave p < 5
-// serves colour pass p: its lane l the colour points t = l + 64 j (j < NT) of
-// each of the BR rows of the pass's current block.  With the pass uniform across the wave, all
-// that depends on it (block, ring slot, rows, colour offset, lhs / rhs row
-// base) is scalar work.  The points t >= 64 NT of each pass (MS of them per
-// row at most) go to spill waves, one point per lane, pass (tid-320) / MS.
+// blocks of BR = 4 or 2 rows) with a fixed lane -> work map.  Wave p < 5 H
+// serves colour pass p % 5, its lane l the colour points t = l + 64 j (j < NT)
+// of each of its rows of the pass's current block: all BR of them with H = 1,
+// half each with H = 2 (FP64 blocks of four rows, sweep_split).  With the pass
+// uniform across the wave, all that depends on it (block, ring slot, rows,
+// colour offset, lhs / rhs row base) is scalar work.  The points t >= 64 NT of
+// each pass (MS of them per row at most) go to spill waves, one point per lane:
+// H runs of waves from thread 320 H on, one for each part of the rows, pass
+// q / MS of lane q of a run.
 // The ring rows have a compile-time
 // stride W >= nni+16, so a point reads its 17 stencil values with immediate
 // offsets from 2 (4/BR) + 1 block bases, and every point of a step is processed
@@ -480,7 +483,9 @@ constexpr int sweep_nsv(int BR) { return sizeof(T) == 4 ? (BR == 4 ? 2 : 1) : 2;
 // pass wave's instructions: with two waves a pass (of two rows each, read
 // together as before) 10 sweeps of 22 potentials of 331 x 601 take 692
 // microseconds, with one 767.  FP32 runs two workgroups side by side, and
-// two-row blocks have no second pair of rows.
+// two-row blocks have no second pair of rows.  (Three waves a SIMD leave 168
+// registers, and 5 or 6 are spilled.)  On 35 batches of 1 .. 150 problems of
+// 61 x 901 .. 331 x 601 the second wave made a call 1.10 to 1.25 times as fast.
 template <typename T>
 __host__ __device__ constexpr int sweep_split(int BR) { return sizeof(T) == 8 && BR == 4 ? 2 : 1; }
 // row stride of k_sweep's padded arrays: nni+8 rounded up to 16 bytes
@@ -1832,8 +1837,10 @@ static int sweep_kind(x2g_ctx *ctx, int maxnni)
 // Kind 4: FP64 problems each resident on a compute unit, all sweeps in one
 // launch.  10 sweeps of 91 x 121 take 110 microseconds so and 313 with a
 // k_sweep launch each, whatever the number of problems up to the compute
-// units'.  Only where all problems of a batch are that small: among large
-// ones they cost a k_sweep launch next to nothing.
+// units' (and beyond: 1500 of 61 x 91 take 724 and took 4690).  Only where all
+// problems of a batch are that small: among large ones they cost a k_sweep
+// launch next to nothing.  Only up to k_sweep's width, so that a grid has one
+// kernel's roundings whether alone or in a batch that k_sweep takes.
 static bool use_resident(x2g_ctx *ctx, int kind, int nni, int nmu)
 {
     return kind == 2 && env_engine() == 0 && env_strip_l() <= 0 && !g_plan_fixed && resident_fits(ctx, nni, nmu);

@@ -25,6 +25,8 @@ waits for a running job to retire.
 Every job's result is independent of which other jobs share its batch: the
 sweeps, quadratures and linear combinations of a job read and write only that
 job's arrays, with a partition of the work that does not depend on the batch.
+(FP64 sweeps have one exception: a grid of more than 336 columns among them
+moves all of a batch's to the kernels for wide grids, whose roundings differ.)
 """
 import contextlib
 import threading

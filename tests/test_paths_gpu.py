@@ -264,3 +264,31 @@ def test_statistics_count_what_ran(shape, kernel, per_launch):
         assert nbytes == word * points * (4 * launches - prec * iters)
         assert ms > 0 and tuple(tot[3 * prec:3 * prec + 3]) == (launches, ms, nbytes) and tot[3 * (1 - prec)] == 0
         p.close()
+
+
+def test_problems_on_grids_of_their_own():
+    """Chains are slower where each problem has a grid of its own and a workgroup
+    holds several: such a batch keeps one launch per sweep, one on a common grid
+    does not, and the results are the same."""
+    from x2dhf_amd import gpu
+    nni, nmu, count = 331, 601, 120
+    res = {}
+    for own in (False, True):
+        print(f"own={own}", flush=True)
+        with gpu.Context(0) as ctx:
+            P = synthetic_problem(nni, nmu, seed=8)
+            grids = [gpu.Grid(ctx, nni, nmu, P["coef"], P["suppl"], P["vxi"], P["veta"])
+                     for _ in range(count if own else 1)]
+            l, r = ctx.upload(P["lhs"]), ctx.upload(P["rhs"])
+            f = ctx.upload(np.tile(P["fun"], count))
+            items = [gpu.RelaxItem(f.ptr + 8 * k * nni * nmu, l.ptr, r.ptr, None, 1.9, (1, -1)[k % 2], 1, 1,
+                                   k if own else 0) for k in range(count)]
+            gh = (gpu._vp * len(grids))(*[g.h.value for g in grids])
+            with Ran(ctx) as ran:
+                gpu.check(ctx.lib.x2g_relax_batch(ctx.h, gh, (gpu.RelaxItem * count)(*items), count, 1, 10))
+            print(ran.n, flush=True)
+            assert ran.kernels == ({"sweep32"} if own else {"chain"})
+            res[own] = f.get().reshape(count, -1)
+            for g in grids:
+                g.destroy()
+    assert np.array_equal(res[False], res[True])

@@ -67,16 +67,29 @@ struct ChainClass {
 // the chip, as the share of the traffic that a step does not hide, and of the
 // memory.  Fitted to 22 and 352 problems of 331 x 601 and 104 of 169 x 241 ..
 // 505 x 901 with 1 .. 4 sweeps per launch and segments of 20 .. 600 rows:
-// within 10 % where the workgroups fill the chip once.  Checked in between, on
-// 118 batches of 1 .. 1500 problems of 61 x 91 .. 505 x 901 (alone and mixed, 1
-// .. 20 sweeps) against one launch per sweep: chains were chosen for 40 of
-// them, 1.01 to 3.1 times as fast, and no batch was slower than it was.
+// within 10 % where the workgroups fill the chip once.
 constexpr double kStepTime = 0.82, kLaunchTime = 8.0, kShareRate = 12.5e6, kChainRate = 4.2e6;
+// Problems alone or few on their grid share no row weights, which then come from
+// memory: steps are longer where problems are alone (0.81 .. 0.91), and hide less
+// traffic where workgroups hold several segments of such grids (0.83 .. 1.19 a
+// step, which the slowest of their waves ends).  Without these two, 120 problems
+// of 331 x 601 on grids of their own took 1443 microseconds in chains and 1256
+// with one launch per sweep.
+//
+// With all of it, 473 calls of 3 .. 1000 problems of 61 x 91 .. 505 x 901 (alone
+// on their grids up to all on one, alone and mixed, 2 .. 15 sweeps) against one
+// launch per sweep: 212 ran as chains, 1.01 to 2.9 times as fast, and none was
+// slower.
+constexpr double kStepLone = 0.05, kShareRateFew = 6.3e6;
+constexpr int kFewProblems = 3;
 // The same for one launch per sweep over the whole batch (k_sweep, as tuned):
 // 25 microseconds, and 224 points per ns on wide grids, 0.75 nni on narrow
 // ones (measured 10 / 45 / 71 / 130 / 168 / 224 / 231 at nni = 19 / 67 / 91 /
 // 163 / 217 / 331 / 505).
 constexpr double kSweepTime = 25.0, kSweepRate = 224e3, kSweepRateNu = 0.75e3;
+// On mixed grids it runs at the stride of the widest, where a row takes what one
+// of the widest grid does: 1.19 ns, more beyond 294 columns.
+static double sweep_row(int maxnni) { return std::max(1.19e-3, maxnni / (200e3 + 160.0 * maxnni)); }
 
 static std::vector<ChainClass> chain_classes(const std::vector<ChainProblem> &probs)
 {
@@ -121,10 +134,16 @@ static double chain_cut(x2g_ctx *ctx, std::vector<ChainClass> &cls, int nsweeps,
         int longest = 1;
         for (auto &c : cls) longest = std::max(longest, chain_steps(2, c.nmu - 3, c.nmu, sw));
         const long whole = wgs(longest);
+        double lone = 0, packs = 0;   // packs, and those of a problem alone on its grid
+        for (auto &c : cls) {
+            packs += c.npack;
+            lone += c.count == 1;
+        }
+        const double step = kStepTime + kStepLone * lone / packs;
         const int r0 = (int)((whole + ctx->num_cu - 1) / ctx->num_cu);
         for (int rounds = r0; rounds < r0 + 2; ++rounds) {
             // least steps with workgroups of `rounds` rounds, where that is a better cut
-            const double room = (best / nch - kLaunchTime) / (rounds * kStepTime);
+            const double room = (best / nch - kLaunchTime) / (rounds * step);
             int lo = 1, hi = (int)std::min<double>(longest, room);
             if (hi < least || wgs(hi) > (long)rounds * ctx->num_cu) continue;
             while (lo < hi) {
@@ -133,11 +152,15 @@ static double chain_cut(x2g_ctx *ctx, std::vector<ChainClass> &cls, int nsweeps,
                 else lo = mid + 1;
             }
             wgs(hi);
-            double bytes = 0;
-            for (auto &c : cls)
-                bytes += (double)c.count * (c.nni - 2) * sizeof(float) *
-                         (4.0 * (c.nmu - 5) + 3.0 * (c.segments() - 1) * (16 + 20 * (sw - 1)));
-            const double t = std::max(rounds * hi * kStepTime + bytes / kShareRate, bytes / kChainRate);
+            double bytes = 0, share = 0;
+            for (auto &c : cls) {
+                const double b = (double)c.count * (c.nni - 2) * sizeof(float) *
+                                 (4.0 * (c.nmu - 5) + 3.0 * (c.segments() - 1) * (16 + 20 * (sw - 1)));
+                const bool several = kChainWaves / (c.wt * sw) > 1;
+                bytes += b;
+                share += b / (several && c.count <= kFewProblems ? kShareRateFew : kShareRate);
+            }
+            const double t = std::max(rounds * hi * step + share, bytes / kChainRate);
             if (nch * (t + kLaunchTime) < best) {
                 best = nch * (t + kLaunchTime);
                 cut = {sw, hi};
@@ -149,11 +172,15 @@ static double chain_cut(x2g_ctx *ctx, std::vector<ChainClass> &cls, int nsweeps,
 
 bool chain_pays(x2g_ctx *ctx, const std::vector<ChainProblem> &probs, int nsweeps, ChainCut &cut)
 {
-    double t = kSweepTime;
+    double t = kSweepTime, rows = 0;
+    int maxnni = 0;
     for (auto &p : probs) {
         if (!chain_fits(p.g->nni, p.g->nmu)) return false;
         t += (double)(p.g->nni - 2) * (p.g->nmu - 5) / std::min(kSweepRate, kSweepRateNu * p.g->nni);
+        rows += p.g->nmu - 5;
+        maxnni = std::max(maxnni, p.g->nni);
     }
+    t = std::max(t, kSweepTime + rows * sweep_row(maxnni));
     std::vector<ChainClass> cls = chain_classes(probs);
     // (less the estimates' errors)
     const double limit = nsweeps * t / 1.08;

@@ -173,9 +173,10 @@ int x2g_set_sweep_engine(int engine, int strip_rows);
  * middle) runs a workgroup per sweep and a thread per column, on grids of 24 x
  * 24 points and more, up to 504 columns where the rows start in the middle and
  * 1016 elsewhere (fewer where the other axis is long: a sweep's row weights lie
- * in LDS); all else, and calls for whose arrays by level there is no memory, run
- * a workgroup per problem on level tables, with one barrier per step of all
- * sweeps.  0 = one dependency level of one sweep per barrier for all
+ * in LDS); all else, calls of a few small problems and several sweeps (below
+ * some 60 x 90 points), where it is the faster one, and calls for whose arrays
+ * by level there is no memory, run a workgroup per problem on level tables, with
+ * one barrier per step of all sweeps.  0 = one dependency level of one sweep per barrier for all
  * (X2G_LEVELS=phase).
  * Each gives the sequential routine's result bit for bit (sormcsor.F90:20-132,
  * 143-386 with one thread).  No counterpart in the reference: a choice of

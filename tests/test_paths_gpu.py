@@ -292,3 +292,47 @@ def test_problems_on_grids_of_their_own():
             for g in grids:
                 g.destroy()
     assert np.array_equal(res[False], res[True])
+
+
+# the smallest fronts, uneven middles; straight, reversed and mirrored orders
+@pytest.mark.parametrize("nni, nmu, method, name", [
+    (24, 24, 1, "col-wise"), (24, 25, 1, "middle"), (25, 24, 2, "col-wise"), (31, 41, 1, "rrow-wis"),
+    (41, 51, 1, "test2"), (45, 67, 1, "test1"),
+])
+def test_small_ordered_grids_take_the_faster_path(nni, nmu, method, name):
+    """Few small problems run several sweeps on the level tables, one sweep as
+    fronts; more problems than CUs, and problems beside a large one, as fronts:
+    bit for bit what the oracle gives."""
+    from x2dhf_amd import gpu
+    code, sweeps, cus = pyoracle.ORDERINGS[name], 20, 256
+    with gpu.Context(0) as ctx:
+        for count, n, beside, kernel in ((1, sweeps, False, "levels"), (6, sweeps, False, "levels"),
+                                         (1, 1, False, "front"), (cus + 1, sweeps, False, "front"),
+                                         (2, sweeps, True, "front")):
+            print(f"{nni}x{nmu} {name} method={method} count={count} sweeps={n} beside={beside}", flush=True)
+            p = Problems(ctx, [(nni, nmu, count, 0, method, code)] + beside * [(121, 161, 1, 0, 1, 1)])
+            with Ran(ctx) as ran:
+                p.relax(1, n)
+            assert ran.kernels == {kernel}, ran.n
+            got = p.get()[0].reshape(count, -1)
+            P, u = synthetic_problem(nni, nmu, seed=70), p.sets[0][1]
+            for k in {0, 1, 2, count - 1} & set(range(count)):
+                it = p.arr[k]
+                w = pyoracle.putin(nni, nmu, it.isym, u[k])
+                pyoracle.relax_ordered(nni, nmu, it.isym, w, P["lhs"], P["rhs"], P["suppl"][it.bkind], P["suppl"][2],
+                                       P["coef"][:16], P["coef"][16:21], it.omega, n, method, name)
+                assert np.array_equal(got[k], pyoracle.putout(nni, nmu, w)), (k, count)
+            p.close()
+        P = synthetic_problem(nni, nmu, seed=3)
+        win = pyoracle.putin(nni, nmu, 1, P["fun"])
+        g = gpu.Grid(ctx, nni, nmu, P["coef"], P["suppl"], P["vxi"], P["veta"])
+        lhs, rhs = ctx.upload(P["lhs"]), ctx.upload(P["rhs"])
+        for n, kernel in ((1, "front"), (sweeps, "levels")):
+            want = pyoracle.relax_ordered(nni, nmu, 1, win.copy(), P["lhs"], P["rhs"], P["suppl"][1], P["suppl"][2],
+                                          P["coef"][:16], P["coef"][16:21], 1.8, n, method, name)
+            w = ctx.upload(win)
+            with Ran(ctx) as ran:
+                gpu.check(ctx.lib.x2g_relax_ordered(g.h, 1, 1, w.ptr, lhs.ptr, rhs.ptr, 1.8, n, method, code))
+            assert ran.kernels == {kernel}, ran.n
+            assert np.array_equal(w.get(), want), n
+        g.destroy()

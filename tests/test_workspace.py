@@ -80,7 +80,7 @@ def test_calls_hold_no_more_than_the_bound(nni, nmu):
 def test_more_sweeps_than_a_launch_of_fronts():
     """2 000 SOR sweeps: two launches of fronts, in the workspace of one."""
     from x2dhf_amd import gpu
-    nni, nmu, sweeps = 24, 25, 2000
+    nni, nmu, sweeps = 61, 91, 2000
     P = synthetic_problem(nni, nmu, seed=2)
     win = pyoracle.putin(nni, nmu, 1, P["fun"])
     with gpu.Context(0) as ctx:

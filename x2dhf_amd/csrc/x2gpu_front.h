@@ -13,8 +13,11 @@ struct FrontItem {
     double omega;
     int bkind, isym, method, ordering;
 };
-// Whether (method, ordering) on a grid of nni x nmu runs as fronts.
+// Whether (method, ordering) on a grid of nni x nmu can run as fronts.
 bool front_fits(const x2g_ctx *ctx, int nni, int nmu, int method, int ordering);
+// Whether nsweeps sweeps of the items (each fits) are faster as fronts than on
+// the level tables.
+bool front_pays(const x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps);
 // Bytes that one problem's fronts add to the workspace at most, however many
 // sweeps (0: does not run as fronts).
 size_t front_workspace_bytes(int nni, int nmu, int method, int ordering);

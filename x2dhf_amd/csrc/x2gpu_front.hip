@@ -423,6 +423,35 @@ bool front_fits(const x2g_ctx *ctx, int nni, int nmu, int method, int ordering)
     return front_fits_lds(ctx->max_lds, nni, nmu, method, ordering);
 }
 
+// The level tables hold a small grid's levels in few steps of one workgroup:
+// there a further sweep costs them less than it costs fronts, whose next sweep
+// follows kReach levels behind.  Microseconds fitted to 440 calls of both, 24 x
+// 24 to 91 x 121 points, 1 to 600 problems, 1 to 40 sweeps (fronts / tables):
+// one of 24 x 24 49 / 82 with 1 sweep, 303 / 181 with 10, 1122 / 525 with 40;
+// of 61 x 91 128 / 259, 392 / 524, 1253 / 1542.  kStepGain is what a front's
+// step saves on the first sweep's, kFrontSweep and kFrontMore a further sweep's
+// time and what each problem beside it adds, the rest the tables' (by latency
+// for few points, by their one workgroup's rate for many).  The choice is the
+// faster one in 431 of the calls and at most 5 % off it in all but one.  The
+// tables' workgroups fill a CU each, so more problems than CUs take turns on
+// them: 600 take fronts 0.27 to 0.98 of the tables' time at every size.
+constexpr double kStepGain = 0.7, kFrontSweep = 30.0, kFrontMore = 0.015;
+constexpr double kTableSweep = 13.0, kTablePoint = 0.003, kTableRate = 170.0;
+
+bool front_pays(const x2g_ctx *ctx, const std::vector<FrontItem> &items, int nsweeps)
+{
+    if ((int)items.size() > ctx->num_cu) return true;
+    // (one that gains decides: the others run beside it)
+    for (auto &it : items) {
+        const double points = (double)it.g->nni * it.g->nmu;
+        const FrontDesc d = front_shape(it.g->nni, it.g->nmu, it.method, it.ordering);
+        const double table = std::max(kTableSweep + kTablePoint * points, points / kTableRate);
+        if (kStepGain * (d.last - kFirst) + nsweeps * (table - kFrontSweep - kFrontMore * items.size()) > 0.0)
+            return true;
+    }
+    return false;
+}
+
 int front_lds_attr(x2g_ctx *ctx)
 {
     const int lds = (int)ctx->max_lds - 64;   // the static part is one word

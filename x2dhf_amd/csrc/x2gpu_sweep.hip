@@ -2987,7 +2987,7 @@ extern "C" int x2g_relax_ordered(x2g_grid *g, int isym, int bkind, double *work_
     if (nsweeps == 0) return X2G_OK;
     if (levels_pipe() && front_fits(g->ctx, g->nni, g->nmu, method, ordering)) {
         const std::vector<FrontItem> fv = {{g, work_d, lhs_d, rhs_d, omega, bkind, isym, method, ordering}};
-        if (front_reserve(g->ctx, fv, nsweeps) == X2G_OK) {
+        if (front_pays(g->ctx, fv, nsweeps) && front_reserve(g->ctx, fv, nsweeps) == X2G_OK) {
             FrontPlan plan;
             if ((rc = set_lds_attr(g->ctx)) || (rc = plan_fronts(g->ctx, fv, nsweeps, plan))) return rc;
             return launch_fronts(g->ctx, plan);
@@ -3267,7 +3267,8 @@ static int relax_batch_eager(x2g_ctx *ctx, x2g_grid *const *grids, const x2g_rel
                               it.method, it.ordering});
         }
     // (level schedules take less memory)
-    if (!fronts.empty() && maxsor2 > 0 && front_reserve(ctx, fronts, maxsor2) != X2G_OK) fronts.clear();
+    if (!front_pays(ctx, fronts, maxsor2) || (maxsor2 > 0 && front_reserve(ctx, fronts, maxsor2) != X2G_OK))
+        fronts.clear();
     const bool fronts_on = !fronts.empty();
     std::vector<PadDesc> pout_ord;
     for (int i : iord) {
